@@ -5,7 +5,9 @@
 // top-left causal mask q_idx >= k_idx within the sequence (:116-119),
 // P cast to the V dtype before P.V (:126), l summing the fp32 P (:128-129).
 //
-// Three kernels, chosen per call:
+// Five kernels, chosen per call:
+//   varlen_prefill_w64   bf16/f16, head_dim 128, GQA group a multiple of 4:
+//                        64 queries per wave (varlen_prefill_w64.h);
 //   varlen_prefill_gqa   bf16/f16, head_dim 64/128, GQA group 2, 4 or 8, up
 //                        to 1024-2048 sequences: persistent workgroups, each
 //                        computing (kv head, sequence, 32 queries) items with
@@ -13,8 +15,10 @@
 //                        MFMA tiles (the main path);
 //   varlen_prefill_mfma  other group sizes: 4 q-heads per workgroup, operands
 //                        straight from global memory, 16x16x32 MFMA tiles;
-//   varlen_prefill_generic  fp32, other head_dims or non-unit innermost
-//                        strides: one wave per (query, q-head), fp32 VALU.
+//   varlen_prefill_f32   fp32, head_dim 64/128: f32 MFMA tiles of 32 (query,
+//                        head) rows (varlen_prefill_f32.hip);
+//   varlen_prefill_generic  other head_dims, non-unit innermost strides or
+//                        unaligned rows: one wave per (query, q-head), VALU.
 // Causal key blocks past a query block's last query are never visited, and
 // the heaviest query blocks are computed first.
 #include <cmath>
@@ -22,6 +26,7 @@
 
 #include "tsa_common.h"
 #include "varlen_prefill_gqa.h"
+#include "varlen_prefill_row.h"
 
 namespace tsa {
 
@@ -182,7 +187,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 template <typename T>
 __global__ __launch_bounds__(64) void varlen_prefill_generic(PrefillArgs a, int64_t total_q) {
   const int64_t qi = blockIdx.x;
-  const int h = blockIdx.y, lane = threadIdx.x;
+  const int h = blockIdx.y;
   // Sequence of query token qi.
   int lo = 0, hi = a.nseq;
   while (hi - lo > 1) {
@@ -194,54 +199,7 @@ __global__ __launch_bounds__(64) void varlen_prefill_generic(PrefillArgs a, int6
   seq_range(a.cu_q, a.cuq_s, b, a.total_q, q_start, q_len);
   seq_range(a.cu_k, a.cuk_s, b, a.total_k, k_start, k_len);
   if (qi < q_start || qi >= q_start + q_len) return;
-  const int64_t qq = qi - q_start;
-  const int kvh = h / a.G, D = a.D;
-  const T* qrow = static_cast<const T*>(a.q) + qi * a.q_st + h * a.q_sh;
-  const T* kb = static_cast<const T*>(a.k) + k_start * a.k_st + kvh * a.k_sh;
-  const T* vb = static_cast<const T*>(a.v) + k_start * a.v_st + kvh * a.v_sh;
-  const int64_t kend = a.causal ? (k_len < qq + 1 ? k_len : qq + 1) : k_len;
-  constexpr int kMaxPerLane = 8;
-  float acc[kMaxPerLane];
-#pragma unroll
-  for (int i = 0; i < kMaxPerLane; ++i) acc[i] = 0.f;
-  float m = kNegInfP, l = 0.f;
-  for (int64_t base = 0; base < kend; base += 64) {
-    const int64_t key = base + lane;
-    float sc = kNegInfP;
-    if (key < kend) {
-      float dot = 0.f;
-      for (int d = 0; d < D; ++d) dot += to_float(qrow[d * a.q_sd]) * to_float(kb[key * a.k_st + d * a.k_sd]);
-      sc = dot * a.scale_log2;
-    }
-    float cmax = sc;
-    for (int off = 32; off >= 1; off >>= 1) cmax = fmaxf(cmax, __shfl_xor(cmax, off, 64));
-    const float m_new = fmaxf(m, cmax);
-    const float alpha = fast_exp2(m - m_new);
-    const float p = fast_exp2(sc - m_new);
-    const float pr = to_float(from_float<T>(p));  // P.V in the V dtype, as the reference does
-    float psum = p;
-    for (int off = 32; off >= 1; off >>= 1) psum += __shfl_xor(psum, off, 64);
-    l = l * alpha + psum;
-#pragma unroll
-    for (int i = 0; i < kMaxPerLane; ++i) acc[i] *= alpha;
-    const int n = static_cast<int>(kend - base < 64 ? kend - base : 64);
-    for (int j = 0; j < n; ++j) {
-      const float pj = __shfl(pr, j, 64);
-      const T* vr = vb + (base + j) * a.v_st;
-#pragma unroll
-      for (int i = 0; i < kMaxPerLane; ++i) {
-        const int d = lane + 64 * i;
-        if (d < D) acc[i] += pj * to_float(vr[d * a.v_sd]);
-      }
-    }
-    m = m_new;
-  }
-  T* orow = static_cast<T*>(a.out) + qi * a.o_st + h * a.o_sh;
-#pragma unroll
-  for (int i = 0; i < kMaxPerLane; ++i) {
-    const int d = lane + 64 * i;
-    if (d < D) orow[d * a.o_sd] = from_float<T>(acc[i] / l);
-  }
+  prefill_row<T>(a, qi, qi - q_start, h, k_start, k_len);
 }
 
 // The persistent kernel runs as many workgroups as fit on the device at once
@@ -285,6 +243,7 @@ template <typename T>
 static int launch_prefill(PrefillArgs& a, bool mfma, int64_t total_q, int64_t max_seqlen_q, hipStream_t stream) {
   if (a.nseq == 0 || a.Hq == 0 || total_q == 0) return TSA_OK;
   if (!mfma) {
+    if (std::is_same<T, float>::value && a.vec16 && prefill_f32_takes(a)) return prefill_f32_launch(a, stream);
     varlen_prefill_generic<T><<<dim3(total_q, a.Hq), dim3(64), 0, stream>>>(a, total_q);
     return check_launch("tsa_varlen_prefill");
   }
@@ -352,8 +311,8 @@ int prefill_prepare(const tsa_view* out, const tsa_view* q, const tsa_view* k, c
   a.total_q = q->size[0]; a.total_k = k->size[0];
   a.causal = causal ? 1 : 0;
   a.scale_log2 = static_cast<float>(softmax_scale * 1.4426950408889634);
-  mfma = (dt == TSA_BF16 || dt == TSA_F16) && (D == 64 || D == 128) && rows_vec16(q) && rows_vec16(k) &&
-         rows_vec16(v) && rows_vec16(out);
+  a.vec16 = rows_vec16(q) && rows_vec16(k) && rows_vec16(v) && rows_vec16(out) ? 1 : 0;
+  mfma = (dt == TSA_BF16 || dt == TSA_F16) && (D == 64 || D == 128) && a.vec16;
   return TSA_OK;
 }
 

@@ -25,7 +25,13 @@ struct PrefillArgs {
   int32_t nseq, Hq, Hkv, G, D, nqb;
   int32_t causal;
   float scale_log2;
+  int32_t vec16;  // q, k, v and out rows are unit-stride and 16-byte aligned (host dispatch)
 };
+
+// varlen_prefill_f32.hip: the float32 kernel, and the calls it takes (vec16
+// rows of 64 or 128 dims).
+bool prefill_f32_takes(const PrefillArgs& a);
+int prefill_f32_launch(const PrefillArgs& a, hipStream_t stream);
 
 // Sequences per call the persistent kernel keeps counts of in LDS.
 constexpr int max_persist_seqs(int nw) { return nw == 2 ? 1024 : 2048; }
