@@ -155,7 +155,10 @@ size_t tsa_paged_decode_workspace_bytes(int64_t num_seqs, int64_t num_heads, int
  * initialisation needed; calls that share one must be ordered on one
  * stream). With num_workgroups 0, a batch of at most 64 (sequence, kv head)
  * units whose tables hold at most 512 tokens takes one launch instead: one
- * workgroup per unit, whose waves merge in LDS and write out. */
+ * workgroup per unit, whose waves merge in LDS and write out. Float32 calls
+ * split each unit over workgroups if the workspace is there, and need none:
+ * without it (NULL, or too small) one workgroup computes a unit, with the
+ * same result. */
 int tsa_paged_decode(const tsa_view* out, const tsa_view* query, const tsa_view* k_cache,
                      const tsa_view* v_cache, const tsa_view* block_tables,
                      const tsa_view* seq_lens, double softmax_scale, void* workspace,
@@ -169,9 +172,9 @@ int tsa_paged_decode(const tsa_view* out, const tsa_view* query, const tsa_view*
  * until the process ends, so it allocates nothing. Every argument is checked
  * before any device work. A call served by the MFMA stream kernel whose
  * workspace (tsa_paged_decode_workspace_bytes) would exceed 16 MiB is then
- * rejected with TSA_ERR_INVALID; calls served by the generic kernel (fp32,
- * other head_dims, more than 16 q-heads per kv head, strided rows) take no
- * scratch and are accepted as tsa_paged_decode accepts them. All calls on one GPU share that
+ * rejected with TSA_ERR_INVALID; float32 calls and calls served by the generic
+ * kernel (other head_dims, more than 16 q-heads per kv head, strided rows)
+ * take no scratch and are accepted as tsa_paged_decode accepts them. All calls on one GPU share that
  * GPU's array: calls ordered on one stream are fine; calls that overlap on
  * one GPU (concurrent streams, threads) race and must not be issued. */
 int tsa_paged_decode_noalloc(const tsa_view* out, const tsa_view* query, const tsa_view* k_cache,

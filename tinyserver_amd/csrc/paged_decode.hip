@@ -58,9 +58,9 @@
 // (the reference would read out of bounds), so a malformed table cannot
 // fault. seq_len == 0 yields NaN, as the reference's 0/0 does.
 //
-// A generic kernel (one wave per (sequence, q-head), fp32 VALU math) covers
-// what the MFMA path does not: fp32 caches, head_dim other than 64/128, GQA
-// groups over 16, non-unit innermost strides.
+// Float32 has its own kernel (paged_decode_f32.hip). A generic kernel (one wave
+// per (sequence, q-head), fp32 VALU math) covers what neither does: head_dim
+// other than 64/128, GQA groups over 16, non-unit innermost strides.
 #include <atomic>
 #include <cmath>
 #include <mutex>
@@ -68,38 +68,10 @@
 
 #include "tsa_common.h"
 #include "norm_rope_row.h"
+#include "paged_decode.h"
 #include "varlen_prefill_gqa.h"
 
 namespace tsa {
-
-struct DecodeArgs {
-  void* out;
-  const void* q;
-  const void* kc;
-  const void* vc;
-  const int32_t* bt;
-  const int32_t* seq_lens;
-  int64_t o_ss, o_sh, o_sd;
-  int64_t q_ss, q_sh, q_sd;
-  int64_t kc_b, kc_h, kc_s, kc_d;
-  int64_t vc_b, vc_h, vc_s, vc_d;
-  int64_t bt_s0, bt_s1, sl_s;
-  int64_t NB;
-  int32_t B, Hq, Hkv, G, BS, max_blocks, D;
-  int32_t W;        // workgroups of the stream kernel
-  int32_t NW;       // wave workers sharing the tile list (kWaves * W)
-  int32_t unit;     // 1: one workgroup per (sequence, kv head) unit, W = B * Hkv, no merge launch
-  float scale_log2;
-  float* part;      // [B * Hkv + NW][G * (D + 2)]: per (unit, worker) acc[G][D], m[G], l[G]
-  int32_t* pref_out;  // [B + 1] tile prefix over the sequences, for the merge
-  // The fused decode step only: query is the raw projection, and the new
-  // token's raw k/v rows (B, Hkv, D), the norm weights (D) and the cos/sin
-  // rows (B, D) come in here; eps is the RMSNorm epsilon.
-  const void* kn; const void* vn; const void* qw; const void* kw; const void* cos; const void* sin;
-  void* kc_out; void* vc_out;  // the caches, written (the new token's rows)
-  int64_t kn_ss, kn_sh, vn_ss, vn_sh, cs_ss, sn_ss;
-  float eps;
-};
 
 template <typename T>
 __device__ __forceinline__ u32x4 pack8(const float (&v)[8]) {
@@ -155,7 +127,6 @@ __device__ __forceinline__ void norm_rope_rows_lds(uint32_t rows, int first, int
 #endif
 constexpr int kWaves = TSA_DECODE_WAVES;
 constexpr int kThreads = 64 * kWaves;
-constexpr float kNegInf = -INFINITY;
 
 // Minimum waves per SIMD the stream kernel is compiled for (register budget:
 // 512 / waves VGPRs per lane), and the number of tiles each wave keeps in
@@ -209,12 +180,6 @@ template <bool NT, typename T>
 __device__ __forceinline__ u32x4 load_stream(const T* p) {
   if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
   else return *reinterpret_cast<const u32x4*>(p);
-}
-
-__device__ __forceinline__ int64_t clamp_len(const DecodeArgs& a, int s) {
-  int64_t L = a.seq_lens[s * a.sl_s];
-  const int64_t cap = static_cast<int64_t>(a.max_blocks) * a.BS;
-  return L < 0 ? 0 : (L > cap ? cap : L);
 }
 
 __device__ __forceinline__ int tiles_of(const DecodeArgs& a, int s) {
@@ -1052,6 +1017,7 @@ template <typename T>
 static int launch_decode(DecodeArgs& a, bool mfma, hipStream_t stream, bool fused = false) {
   if (a.B == 0 || a.Hq == 0) return TSA_OK;
   if (!mfma) {
+    if (a.S > 0) return decode_f32_launch(a, stream);  // (float32 only)
     paged_decode_generic<T><<<dim3(a.Hq, a.B), dim3(64), 0, stream>>>(a);
     return check_launch("tsa_paged_decode");
   }
@@ -1185,15 +1151,27 @@ static int check_decode(const tsa_view* out, const tsa_view* query, const tsa_vi
     a.W = plan.W;
     a.NW = kWaves * plan.W;
     a.unit = plan.unit ? 1 : 0;
+  } else if (dt == TSA_F32 && rows_vec16(query) && rows_vec16(k_cache) && rows_vec16(v_cache) && decode_f32_takes(a)) {
+    // The partials of its splits fit the plan's slots, so the workspace the
+    // caller was told to bring serves (the one-workgroup-per-unit form has no
+    // slots: one split).
+    plan = make_plan(B, Hq, Hkv, D, block_tables->size[1], BS, num_workgroups);
+    const int64_t units = B * Hkv;
+    a.S = units == 0 ? 1 : decode_f32_splits(units, (block_tables->size[1] * BS + 15) / 16,
+                                             plan.unit ? 0 : units + static_cast<int64_t>(kWaves) * plan.W);
   }
   return TSA_OK;
 }
 
-// The stream kernel's partials and tile prefix in the workspace (only the
-// stream path takes one).
+// The stream kernel's partials and tile prefix in the workspace. Float32
+// calls need none: without one that fits, one workgroup computes a unit.
 static int bind_workspace(DecodeArgs& a, bool mfma, const DecodePlan& plan, void* workspace, size_t workspace_bytes,
                           const char* workspace_name) {
-  if (!mfma) return TSA_OK;
+  if (!mfma) {
+    if (a.S > 1 && workspace != nullptr && workspace_bytes >= plan.total && reinterpret_cast<uintptr_t>(workspace) % 4 == 0)
+      a.part = static_cast<float*>(workspace);
+    return TSA_OK;
+  }
   TSA_REQUIRE(workspace != nullptr && workspace_bytes >= plan.total, "%s of %zu bytes is too small: %zu needed",
               workspace_name, workspace_bytes, plan.total);
   TSA_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 256 == 0, "%s must be 256-byte aligned", workspace_name);

@@ -123,10 +123,12 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
   seq_range(a.cu_q, a.cuq_s, b, a.total_q, q_start, q_len);
   seq_range(a.cu_k, a.cuk_s, b, a.total_k, k_start, k_len);
   const int G = a.G;
-  const int64_t row0 = static_cast<int64_t>(tile) * kF32Rows, n_rows = q_len * G;
-  const int rows = static_cast<int>(n_rows - row0 < kF32Rows ? n_rows - row0 : kF32Rows);
+  // (32-bit rows: the host takes calls of fewer than 2^31 rows)
+  const uint32_t row0 = static_cast<uint32_t>(tile) * kF32Rows, n_rows = static_cast<uint32_t>(q_len) * G;
+  const int rows = static_cast<int>(min(n_rows - row0, static_cast<uint32_t>(kF32Rows)));
   // Row r of the item: query (row0 + r) / G, q-head kvh G + (row0 + r) % G.
-  auto q_of = [&](int r) { return static_cast<int>((row0 + r) / G); };
+  auto q_of = [&](int r) { return static_cast<int>((row0 + r) / static_cast<uint32_t>(G)); };
+  auto head_of = [&](int r, int qq) { return kvh * G + static_cast<int>(row0 + r - static_cast<uint32_t>(qq) * G); };
   const int q_first = q_of(0), q_last = q_of(rows - 1);
   const int kl = static_cast<int>(k_len);
   const int kend = a.causal ? min(kl, q_last + 1) : kl;
@@ -139,8 +141,7 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
   for (int i = tid; i < kF32Rows * (D / 4); i += kF32Threads) {
     const int r = i / (D / 4), ch = i - r * (D / 4);
     const int rr = min(r, rows - 1), qq = q_of(rr);
-    const int hd = static_cast<int>(row0 + rr - static_cast<int64_t>(qq) * G);
-    const float* src = static_cast<const float*>(a.q) + (q_start + qq) * a.q_st + (kvh * G + hd) * a.q_sh + 4 * ch;
+    const float* src = static_cast<const float*>(a.q) + (q_start + qq) * a.q_st + head_of(rr, qq) * a.q_sh + 4 * ch;
     *reinterpret_cast<f32x4*>(smem + r * RP + 4 * ch) = *reinterpret_cast<const f32x4*>(src);
   }
 
@@ -175,6 +176,7 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
       }
     };
     load_v(0);
+    __builtin_amdgcn_sched_barrier(0);  // in flight under the score products
     f32x16v sc;
 #pragma unroll
     for (int e = 0; e < 16; ++e) sc[e] = 0.f;
@@ -186,6 +188,7 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
       for (int i = 0; i < 4; ++i) sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kop[j][i], qv[i], sc, 0, 0, 0);
     }
     load_v(8);
+    __builtin_amdgcn_sched_barrier(0);
 
     float s[16];
     const bool edge = k0 + 32 > full;  // some row does not see some key of the block
@@ -201,9 +204,9 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
     for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[e]);
     mx = fmaxf(mx, __builtin_bit_cast(float, xor_lane32<32>(__builtin_bit_cast(uint32_t, mx), lane)));
     const float m_new = fmaxf(m, mx);
-    const bool any = m_new != kNegInfP;  // false: row c sees no key yet
+    const float mu = m_new == kNegInfP ? 0.f : m_new;  // (-inf: every score of row c so far is -inf, and weighs 0)
     if (__any(m_new > m)) {
-      const float alpha = any ? fast_exp2(m - m_new) : 1.f;
+      const float alpha = fast_exp2(m - mu);
       l *= alpha;
 #pragma unroll
       for (int u = 0; u < NU; ++u)
@@ -213,7 +216,7 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
     }
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      s[e] = any ? fast_exp2(s[e] - m) : 0.f;
+      s[e] = fast_exp2(s[e] - mu);
       l += s[e];
     }
     // A key that some row does not see must not reach that row: its weight is
@@ -238,6 +241,7 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
     // The next block's K, into the registers that V's first half leaves
     // (the wave's last block loads itself again).
     load_k(min(blk + 4, nblk - 1));
+    __builtin_amdgcn_sched_barrier(0);  // under the second half of P V
     pv(8);
   }
   l += __builtin_bit_cast(float, xor_lane32<32>(__builtin_bit_cast(uint32_t, l), lane));
@@ -245,8 +249,7 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
   if (__syncthreads_or(bad)) {
     for (int r = wave; r < rows; r += 4) {
       const int qq = q_of(r);
-      prefill_row<float>(a, q_start + qq, qq, kvh * G + static_cast<int>(row0 + r - static_cast<int64_t>(qq) * G),
-                         k_start, k_len);
+      prefill_row<float>(a, q_start + qq, qq, head_of(r, qq), k_start, k_len);
     }
     return;
   }
@@ -284,8 +287,8 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
 #pragma unroll
       for (int x = 0; x < 4; ++x) o[x] += f * p[x];
     }
-    const int qq = q_of(r), hd = static_cast<int>(row0 + r - static_cast<int64_t>(qq) * G);
-    float* dst = static_cast<float*>(a.out) + (q_start + qq) * a.o_st + (kvh * G + hd) * a.o_sh + 4 * ch;
+    const int qq = q_of(r);
+    float* dst = static_cast<float*>(a.out) + (q_start + qq) * a.o_st + head_of(r, qq) * a.o_sh + 4 * ch;
 #pragma unroll
     for (int x = 0; x < 4; ++x) o[x] /= den;
     *reinterpret_cast<f32x4*>(dst) = o;
