@@ -2,34 +2,37 @@
 //
 // Reference: server/model/kernels/varlen_attention.py:8-142.
 //
-// What bounds it: v_mfma_f32_32x32x2_f32, 64 cycles for 4,096 FLOP a SIMD (a
-// large float32 matrix product reaches 133 TFLOP/s on this card), so the
-// kernel keeps that pipe fed and nothing else matters much: the operands come
-// straight from global memory (the L2 after the first touch) into registers,
-// a K/V block of 32 keys feeding 128 instructions, 8,192 cycles.
+// What bounds it: v_mfma_f32_16x16x4_f32, 32 cycles for 2,048 FLOP a SIMD (a
+// large float32 matrix product reaches 133 TFLOP/s on this card; one
+// 8192-token sequence of 16/8 heads, 275 GFLOP, runs at 121 here). Small
+// batches are bound by the items' serial parts -- the search, the first loads
+// and the merge, about 7 us a workgroup, of which two share a CU: 8 prompts of
+// 32-512 tokens, 3.5 GFLOP, take 58 us where the products alone need 26.
+// (The one-wave-per-row kernel took 3,355.)
 //
 // Work item: 32 rows of one (sequence, kv head), a row being one (query,
 // q-head of the kv head's group), query-major, so one K/V read serves the
 // whole GQA group and a tile spans only 32 / G queries of the causal diagonal.
-// One 4-wave workgroup takes an item and deals its 32-key blocks to the waves
+// One 4-wave workgroup takes an item and deals its 16-key blocks to the waves
 // in turn: short items then finish in a quarter of the time one wave would
 // take, which is what fills 1,024 SIMDs from a few thousand tokens. The waves'
 // partials (m, l, O^T) meet in LDS once per item. Two workgroups share a CU
-// (68 KB of LDS each, at most 256 registers a wave).
+// (at most 256 registers a wave). K and V come from global memory (the L2
+// after the first touch) straight into registers: V is in flight under the
+// score products, the next block's K under the softmax and P V. Blocks of 32
+// keys on the 32x32x2 form took 68 us for that batch (coarser blocks to deal,
+// more masked work); workgroups that stay and walk a precomputed item plan
+// took 59, and 2,430 against 2,264 for the long sequence.
 //
-// Layouts. With lane (h, c) = (lane / 32, lane % 32):
-//   S^T(32 keys x 32 rows) = K Q^T: step 4 J + i takes dims 8 J + 4 h + i, so a
-//     lane's K and Q operands are 16-byte pieces of key c's and row c's vectors;
-//     element e of the accumulator is the score of key 8 (e/4) + 4 h + e%4 for
-//     row c.
-//   O^T(dims x rows) += V^T P^T: step e takes keys 8 (e/4) + e%4 (+ 4 for h = 1),
-//     whose probabilities are element e of the scores' lanes: P never leaves its
-//     registers. Tile u's row r is dim NU r + u, so a lane's V operands of a key
-//     are NU consecutive floats. A lane holds row c's outputs, so the softmax's
-//     scales are the lane's own.
-//
-// Measured: 8 prompts of 32-512 tokens, 16/8 heads of 128 dims
-// (perf case sizes, 3.5 GFLOP): see kept figures at the launch below.
+// Layouts. With lane (g, c) = (lane / 16, lane % 16) and row tiles t = 0, 1:
+//   S^T(16 keys x 16 rows) = K Q^T: step 4 j + i takes dims 16 j + 4 g + i, so
+//     a lane's K and Q operands are 16-byte pieces of key c's and row c's
+//     vectors; element r of the accumulator is the score of key 4 g + r.
+//   O^T(dims x 16 rows) += V^T P^T: step r takes keys 4 g + r, whose weights are
+//     element r of the lane's own scores: P never leaves its registers. Dim
+//     tile (y, i) has dim 64 y + 4 c + i in its row c, so a lane's V operands
+//     are 16-byte pieces of a key's row. A lane holds row c's outputs, so the
+//     softmax's scales are the lane's own.
 #include <cmath>
 
 #include "tsa_common.h"
@@ -40,8 +43,6 @@ namespace tsa {
 
 constexpr int kF32Rows = 32;     // rows of an item
 constexpr int kF32Threads = 256;
-
-typedef float f32x16v __attribute__((ext_vector_type(16)));
 
 // Tiles of 32 (query, head-of-group) rows of sequence b.
 __device__ __forceinline__ int f32_tiles(const PrefillArgs& a, int b) {
@@ -101,20 +102,21 @@ __device__ __forceinline__ bool f32_item(const PrefillArgs& a, int j, int& b, in
 
 template <int D>
 constexpr int f32_row_floats() { return D + 4; }  // LDS row pitch: 16-byte aligned, rows 4 banks apart
+// LDS: three waves' partials (Q's rows sit in the first until the merge) and
+// all four waves' m and l.
 template <int D>
-constexpr int f32_smem_floats() { return 4 * kF32Rows * f32_row_floats<D>() + 2 * 4 * kF32Rows; }
+constexpr int f32_smem_floats() { return 3 * kF32Rows * f32_row_floats<D>() + 2 * 4 * kF32Rows; }
 
 template <int D>
 __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 2))) void varlen_prefill_f32(
     PrefillArgs a) {
-  constexpr int NJ = D / 8;   // 16-byte pieces of a lane's K or Q operand
-  constexpr int NU = D / 32;  // output tiles: consecutive dims a lane reads of a V row
+  constexpr int NJ = D / 16;  // 16-byte pieces of a lane's K or Q operand
+  constexpr int NH = D / 64;  // 16-byte pieces of a lane's V operand of one key
   constexpr int RP = f32_row_floats<D>();
-  typedef float vrow_t __attribute__((ext_vector_type(NU)));
   __shared__ __align__(16) float smem[f32_smem_floats<D>()];
-  float* const ml = smem + 4 * kF32Rows * RP;  // m[4][32], l[4][32]
+  float* const ml = smem + 3 * kF32Rows * RP;  // m[4][32], l[4][32]
 
-  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, c = lane & 31;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kvh = static_cast<int>(blockIdx.x) % a.Hkv;
   int b, tile;
@@ -132,10 +134,8 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
   const int q_first = q_of(0), q_last = q_of(rows - 1);
   const int kl = static_cast<int>(k_len);
   const int kend = a.causal ? min(kl, q_last + 1) : kl;
-  const int nblk = (kend + 31) / 32;
+  const int nblk = (kend + 15) / 16;
   const int full = a.causal ? min(kl, q_first + 1) : kl;  // keys below it are seen by every row
-  const int my_q = q_of(min(c, rows - 1));
-  const int my_end = a.causal ? min(kl, my_q + 1) : kl;    // keys row c sees
 
   // The item's Q rows into LDS (rows past the last repeat it).
   for (int i = tid; i < kF32Rows * (D / 4); i += kF32Threads) {
@@ -145,79 +145,89 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
     *reinterpret_cast<f32x4*>(smem + r * RP + 4 * ch) = *reinterpret_cast<const f32x4*>(src);
   }
 
-  const float* const kb = static_cast<const float*>(a.k) + k_start * a.k_st + kvh * a.k_sh + 4 * h;
-  const float* const vb = static_cast<const float*>(a.v) + k_start * a.v_st + kvh * a.v_sh + NU * c;
+  const float* const kb = static_cast<const float*>(a.k) + k_start * a.k_st + kvh * a.k_sh + 4 * g;
+  const float* const vb = static_cast<const float*>(a.v) + k_start * a.v_st + kvh * a.v_sh + 4 * c;
   f32x4 kop[NJ];
   // Keys past the sequence's last re-read it; their scores are masked.
   auto load_k = [&](int blk) __attribute__((always_inline)) {
-    const float* p = kb + static_cast<int64_t>(min(blk * 32 + c, kl - 1)) * a.k_st;
+    const float* p = kb + static_cast<int64_t>(min(blk * 16 + c, kl - 1)) * a.k_st;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) kop[j] = *reinterpret_cast<const f32x4*>(p + 8 * j);
+    for (int j = 0; j < NJ; ++j) kop[j] = *reinterpret_cast<const f32x4*>(p + 16 * j);
   };
   if (wave < nblk) load_k(wave);
+  int my_end[2];  // keys that rows c and 16 + c see
+#pragma unroll
+  for (int t = 0; t < 2; ++t) my_end[t] = a.causal ? min(kl, q_of(min(16 * t + c, rows - 1)) + 1) : kl;
   __syncthreads();
 
-  float m = kNegInfP, l = 0.f;
+  float m[2] = {kNegInfP, kNegInfP}, l[2] = {0.f, 0.f};
   bool bad = false;
-  f32x16v acc[NU];
+  f32x4 acc[2][NH][4];
 #pragma unroll
-  for (int u = 0; u < NU; ++u)
+  for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[u][e] = 0.f;
+    for (int y = 0; y < NH; ++y)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[t][y][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   for (int blk = wave; blk < nblk; blk += 4) {
-    const int k0 = blk * 32;
-    vrow_t vop[16];
-    auto load_v = [&](int e0) __attribute__((always_inline)) {  // eight of the lane's sixteen V operands
+    const int k0 = blk * 16;
+    f32x4 vop[4][NH];
 #pragma unroll
-      for (int e = e0; e < e0 + 8; ++e) {
-        const int key = min(k0 + 8 * (e / 4) + 4 * h + e % 4, kl - 1);
-        vop[e] = *reinterpret_cast<const vrow_t*>(vb + static_cast<int64_t>(key) * a.v_st);
-      }
-    };
-    load_v(0);
+    for (int r = 0; r < 4; ++r) {
+      const float* p = vb + static_cast<int64_t>(min(k0 + 4 * g + r, kl - 1)) * a.v_st;
+#pragma unroll
+      for (int y = 0; y < NH; ++y) vop[r][y] = *reinterpret_cast<const f32x4*>(p + 64 * y);
+    }
     __builtin_amdgcn_sched_barrier(0);  // in flight under the score products
-    f32x16v sc;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) sc[e] = 0.f;
-    const float* qrow = smem + c * RP + 4 * h;
+    f32x4 sc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    const float* qrow = smem + c * RP + 4 * g;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-      const f32x4 qv = *reinterpret_cast<const f32x4*>(qrow + 8 * j);
+      const f32x4 q0 = *reinterpret_cast<const f32x4*>(qrow + 16 * j);
+      const f32x4 q1 = *reinterpret_cast<const f32x4*>(qrow + 16 * RP + 16 * j);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kop[j][i], qv[i], sc, 0, 0, 0);
+      for (int i = 0; i < 4; ++i) {
+        sc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kop[j][i], q0[i], sc[0], 0, 0, 0);
+        sc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kop[j][i], q1[i], sc[1], 0, 0, 0);
+      }
     }
-    load_v(8);
-    __builtin_amdgcn_sched_barrier(0);
+    load_k(min(blk + 4, nblk - 1));     // the wave's next block (its last: a repeat)
+    __builtin_amdgcn_sched_barrier(0);  // in flight under the softmax and P V
 
-    float s[16];
-    const bool edge = k0 + 32 > full;  // some row does not see some key of the block
+    const bool edge = k0 + 16 > full;  // some row does not see some key of the block
+    float p[2][4];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) s[e] = sc[e] * a.scale_log2;
-    if (edge) {
+    for (int t = 0; t < 2; ++t) {
+      float s[4];
 #pragma unroll
-      for (int e = 0; e < 16; ++e)
-        if (k0 + 8 * (e / 4) + 4 * h + e % 4 >= my_end) s[e] = kNegInfP;
-    }
-    float mx = s[0];
+      for (int r = 0; r < 4; ++r) s[r] = sc[t][r] * a.scale_log2;
+      if (edge) {
 #pragma unroll
-    for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[e]);
-    mx = fmaxf(mx, __builtin_bit_cast(float, xor_lane32<32>(__builtin_bit_cast(uint32_t, mx), lane)));
-    const float m_new = fmaxf(m, mx);
-    const float mu = m_new == kNegInfP ? 0.f : m_new;  // (-inf: every score of row c so far is -inf, and weighs 0)
-    if (__any(m_new > m)) {
-      const float alpha = fast_exp2(m - mu);
-      l *= alpha;
+        for (int r = 0; r < 4; ++r)
+          if (k0 + 4 * g + r >= my_end[t]) s[r] = kNegInfP;
+      }
+      float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+      mx = fmaxf(mx, __builtin_bit_cast(float, xor_lane32<16>(__builtin_bit_cast(uint32_t, mx), lane)));
+      mx = fmaxf(mx, __builtin_bit_cast(float, xor_lane32<32>(__builtin_bit_cast(uint32_t, mx), lane)));
+      const float m_new = fmaxf(m[t], mx);
+      const float mu = m_new == kNegInfP ? 0.f : m_new;  // (-inf: every score of the row so far is -inf, and weighs 0)
+      if (__any(m_new > m[t])) {
+        const float alpha = fast_exp2(m[t] - mu);
+        l[t] *= alpha;
 #pragma unroll
-      for (int u = 0; u < NU; ++u)
+        for (int y = 0; y < NH; ++y)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[u][e] *= alpha;
-      m = m_new;
-    }
+          for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      s[e] = fast_exp2(s[e] - mu);
-      l += s[e];
+            for (int e = 0; e < 4; ++e) acc[t][y][i][e] *= alpha;
+        m[t] = m_new;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        p[t][r] = fast_exp2(s[r] - mu);
+        l[t] += p[t][r];
+      }
     }
     // A key that some row does not see must not reach that row: its weight is
     // 0, but 0 times an infinity or NaN in its V row is NaN. An item that
@@ -225,26 +235,28 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
     if (edge) {
       float z = 0.f;
 #pragma unroll
-      for (int e = 0; e < 16; ++e)
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int u = 0; u < NU; ++u) z = fmaf(vop[e][u], 0.f, z);
+        for (int y = 0; y < NH; ++y)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) z = fmaf(vop[r][y][i], 0.f, z);
       bad |= z != 0.f;  // NaN
     }
-    auto pv = [&](int e0) __attribute__((always_inline)) {
 #pragma unroll
-      for (int e = e0; e < e0 + 8; ++e)
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int u = 0; u < NU; ++u)
-          acc[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(vop[e][u], s[e], acc[u], 0, 0, 0);
-    };
-    pv(0);
-    // The next block's K, into the registers that V's first half leaves
-    // (the wave's last block loads itself again).
-    load_k(min(blk + 4, nblk - 1));
-    __builtin_amdgcn_sched_barrier(0);  // under the second half of P V
-    pv(8);
+      for (int y = 0; y < NH; ++y)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          acc[0][y][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vop[r][y][i], p[0][r], acc[0][y][i], 0, 0, 0);
+          acc[1][y][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vop[r][y][i], p[1][r], acc[1][y][i], 0, 0, 0);
+        }
   }
-  l += __builtin_bit_cast(float, xor_lane32<32>(__builtin_bit_cast(uint32_t, l), lane));
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    l[t] += __builtin_bit_cast(float, xor_lane32<16>(__builtin_bit_cast(uint32_t, l[t]), lane));
+    l[t] += __builtin_bit_cast(float, xor_lane32<32>(__builtin_bit_cast(uint32_t, l[t]), lane));
+  }
 
   if (__syncthreads_or(bad)) {
     for (int r = wave; r < rows; r += 4) {
@@ -254,44 +266,54 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
     return;
   }
 
-  // The four waves' partials meet in LDS (Q is no longer read).
-  float* const mine = smem + (wave * kF32Rows + c) * RP;
+  // The waves' partials: waves 1 to 3 leave theirs in LDS (Q is no longer
+  // read), wave 0 adds them to its registers and writes the rows.
+  // Element e of acc[t][y][i] is row 16 t + c, dim 64 y + 4 (4 g + e) + i.
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    vrow_t o;
+  for (int t = 0; t < 2; ++t)
+    if (g == 0) {
+      ml[wave * kF32Rows + 16 * t + c] = m[t];
+      ml[(4 + wave) * kF32Rows + 16 * t + c] = l[t];
+    }
+  if (wave > 0) {
 #pragma unroll
-    for (int u = 0; u < NU; ++u) o[u] = acc[u][e];
-    *reinterpret_cast<vrow_t*>(mine + NU * (8 * (e / 4) + 4 * h + e % 4)) = o;
-  }
-  if (h == 0) {
-    ml[wave * kF32Rows + c] = m;
-    ml[(4 + wave) * kF32Rows + c] = l;
+    for (int t = 0; t < 2; ++t) {
+      float* const mine = smem + ((wave - 1) * kF32Rows + 16 * t + c) * RP + 16 * g;
+#pragma unroll
+      for (int y = 0; y < NH; ++y)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          *reinterpret_cast<f32x4*>(mine + 64 * y + 4 * e) =
+              f32x4{acc[t][y][0][e], acc[t][y][1][e], acc[t][y][2][e], acc[t][y][3][e]};
+    }
   }
   __syncthreads();
-  for (int i = tid; i < rows * (D / 4); i += kF32Threads) {
-    const int r = i / (D / 4), ch = i - r * (D / 4);
-    float mw[4], M = kNegInfP;
+  if (wave > 0) return;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int r = 16 * t + c;
+    float f[4], M = kNegInfP, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) M = fmaxf(M, ml[w * kF32Rows + r]);
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-      mw[w] = ml[w * kF32Rows + r];
-      M = fmaxf(M, mw[w]);
+      const float mw = ml[w * kF32Rows + r];
+      f[w] = mw == kNegInfP ? 0.f : fast_exp2(mw - M);  // (a wave without a seen key: l = 0 and O = 0)
+      den = fmaf(f[w], ml[(4 + w) * kF32Rows + r], den);
     }
-    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
-    float den = 0.f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float f = mw[w] == kNegInfP ? 0.f : fast_exp2(mw[w] - M);
-      // A wave without a seen key has l = 0 and O = 0, and weighs nothing.
-      den += f * ml[(4 + w) * kF32Rows + r];
-      const f32x4 p = *reinterpret_cast<const f32x4*>(smem + (w * kF32Rows + r) * RP + 4 * ch);
-#pragma unroll
-      for (int x = 0; x < 4; ++x) o[x] += f * p[x];
-    }
+    if (r >= rows) continue;
     const int qq = q_of(r);
-    float* dst = static_cast<float*>(a.out) + (q_start + qq) * a.o_st + head_of(r, qq) * a.o_sh + 4 * ch;
+    float* const dst = static_cast<float*>(a.out) + (q_start + qq) * a.o_st + head_of(r, qq) * a.o_sh + 16 * g;
 #pragma unroll
-    for (int x = 0; x < 4; ++x) o[x] /= den;
-    *reinterpret_cast<f32x4*>(dst) = o;
+    for (int y = 0; y < NH; ++y)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f32x4 o = f32x4{acc[t][y][0][e], acc[t][y][1][e], acc[t][y][2][e], acc[t][y][3][e]} * f[0];
+#pragma unroll
+        for (int w = 1; w < 4; ++w)
+          o += *reinterpret_cast<const f32x4*>(smem + ((w - 1) * kF32Rows + r) * RP + 64 * y + 16 * g + 4 * e) * f[w];
+        *reinterpret_cast<f32x4*>(dst + 64 * y + 4 * e) = o / den;
+      }
   }
 }
 
