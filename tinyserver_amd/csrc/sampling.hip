@@ -37,8 +37,18 @@
 // only the few elements above that bound are gathered, ranked and decided
 // on. A row it cannot finish (too many candidates, NaN or inf) continues down
 // the paths above.
+//
+// bf16 rows of 16,384 to 155,648 logits then take the key-count pass
+// (RowSampler::by_keys): a bf16 row has few distinct values, so one LDS count
+// per value settles every decision, with no mass atomics, no gather and no
+// sort, and no second launch. Measured against the split launches below, which
+// it replaces for these rows (151,936 logits): 64 rows at the server's default
+// request 47 -> 28 us, 8 mixed rows 36 -> 26, 256 rows 103 -> 38, rows of one
+// value 995 -> 147; top-k and greedy rows, which needed neither launch, 17 ->
+// 13 (eager).
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include "tsa_common.h"
 
@@ -62,6 +72,7 @@ struct SampleArgs {
   const float* unif; int64_t unif_s;
   int64_t* out; int64_t out_s;
   int cand;  // 1: top-k and greedy rows may take the register-resident candidate pass
+  int keys;  // 1: the rows may take the key-count pass (the launch's LDS holds KeyLds)
   // Rows split over S workgroups (split_row; S = 0: none): per (row,
   // segment) the statistics record and the partial histogram, as the
   // exclusive prefix of its counts (plp) and its masses (pmass); with
@@ -334,7 +345,35 @@ struct SampleLds {
   uint64_t found_cum;
   int64_t found_index;
   float found_x;
+  // the row's statistics, per wave (all LDS is in this block, at address 0:
+  // an LDS address is then an index times its size, with no base to add)
+  float red_mx[kSampWaves], red_mn[kSampWaves], red_fm[kSampWaves];
+  int red_imx[kSampWaves], red_imn[kSampWaves], red_nan[kSampWaves];
 };
+
+// ---- The key-count pass (bf16 rows that fit the registers): LDS. Bin i
+// counts the elements whose key is i below the row's largest. The keys within
+// 41 binary orders of the maximum are at most about 34,000 (logits up to 2^8
+// either side of 0); a row that needs more than kKeyBins goes on. f16 needs
+// 38,000 to 42,000 at ordinary scales, more than the LDS has words: with two
+// 16-bit counts a word it took 54 us where the split launches take 46 (64
+// rows, the server's default request), so f16 rows stay with those.
+constexpr int64_t kKeysMinV = 16384;  // shorter rows take the histogram path
+constexpr int kKeyBins = 36864;
+constexpr int kKeyBlocks = kSampThreads;  // blocks of 64 bins, one per thread
+struct KeyLds {
+  uint32_t bins[kKeyBins];
+  uint64_t bmass[kKeyBlocks];  // per block: the mass and number of its elements
+  uint32_t bcnt[kKeyBlocks];
+  uint64_t wave_m[kSampWaves];
+  uint32_t wave_c[kSampWaves], wave_x[kSampWaves];
+  uint64_t place_m[3];  // per decision: RowSampler::by_keys's Place
+  uint32_t place_rank[3], place_key[3], place_nth[3];
+  uint32_t token;
+  uint32_t match[kRegChunks * kSampWaves];  // per (chunk span, wave): elements with the picked key
+};
+static_assert(kKeyBlocks * 64 >= kKeyBins, "every bin has a block");
+static_assert(sizeof(KeyLds) <= 160 * 1024 - 1024, "the key-count pass fits a CU's LDS");
 
 template <typename T, bool UNIT>  // UNIT: the row's elements are adjacent (stride 1)
 struct RowSampler {
@@ -1214,6 +1253,295 @@ struct RowSampler {
     return s.found_index;
   }
 
+  // The key-count pass, for a row of bf16 logits in registers (load_row) at
+  // temperature t. All elements of one key (one 16-bit value) weigh the same,
+  // so the count of every key settles all three decisions: a running mass at
+  // any rank is a sum of count x mass_of(key), the same integers that the
+  // histogram paths add up element by element, compared with the same targets.
+  //   1. the row's largest and smallest key (NaN and infinite rows go on);
+  //   2. a count per key in LDS, one 32-bit atomic for each element whose
+  //      mass is not 0 (an element 2^-40 below the maximum weighs nothing, as
+  //      everywhere here; so a row masked with -inf or a lowest value counts
+  //      only what is left);
+  //   3. count and mass of each block of 64 keys, and a scan over the blocks
+  //      (one a thread, descending keys: rank order);
+  //   4. per decision: the block, then the key (one a lane), then the place
+  //      among the key's equal elements where it falls, by the one wave
+  //      that holds the block;
+  //   5. the token: the nth element, in index order, with the pick's key
+  //      (counted per span of 1,024 chunks and wave, then one wave's lanes).
+  // One workgroup reads the row once, makes one atomic an element and sorts
+  // nothing. It is bound by the 16 waves' instructions per element (one
+  // vector instruction an element costs the CU 2,400 cycles, 1 us), hence the
+  // packed forms. The token, or -1 to send the row on.
+  __device__ __forceinline__ int64_t by_keys(u32x4 (&ch)[kRegChunks], KeyLds& q, int64_t k, double p, double u) {
+    const int n8 = static_cast<int>(a.V >> 3);
+    lds_barrier();  // (the candidate pass may have used this LDS; the row may still be in flight)
+    u32x4* const bins4 = reinterpret_cast<u32x4*>(q.bins);
+#pragma unroll
+    for (int i = 0; i < kKeyBins / 4 / kSampThreads; ++i) bins4[i * kSampThreads + tid] = u32x4{0, 0, 0, 0};
+    static_assert(kKeyBins % (4 * kSampThreads) == 0, "whole rounds of 16 bytes a thread clear the bins");
+    q.bcnt[tid] = 0;
+    q.bmass[tid] = 0;
+    if (tid < 3) q.place_rank[tid] = 0;  // (a place found has rank 1 or more)
+    __builtin_amdgcn_sched_barrier(0);   // cleared while the row arrives
+    // 1. (a clamped load repeats chunks, which leaves the extremes as they are)
+    uint32_t mx = 0, mn = 0xFFFFFFFFu;
+#pragma unroll
+    for (int j = 0; j < kRegChunks; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        ch[j][e] = pk_key(ch[j][e]);
+        mx = pk_max(mx, ch[j][e]);
+        mn = pk_min(mn, ch[j][e]);
+      }
+    uint32_t ext = hmax(mx) | ((0xFFFFu - min(mn & 0xFFFFu, mn >> 16)) << 16);  // packed: max, 0xFFFF - min
+    ext = pk_max(ext, xor_lane32<1>(ext, lane));
+    ext = pk_max(ext, xor_lane32<2>(ext, lane));
+    ext = pk_max(ext, xor_lane32<4>(ext, lane));
+    ext = pk_max(ext, xor_lane32<8>(ext, lane));
+    ext = pk_max(ext, xor_lane32<16>(ext, lane));
+    ext = pk_max(ext, xor_lane32<32>(ext, lane));
+    if (lane == 0) q.wave_x[wave] = ext;
+    lds_barrier();
+    ext = q.wave_x[lane & (kSampWaves - 1)];
+    ext = pk_max(ext, xor_lane32<1>(ext, lane));
+    ext = pk_max(ext, xor_lane32<2>(ext, lane));
+    ext = pk_max(ext, xor_lane32<4>(ext, lane));
+    ext = pk_max(ext, xor_lane32<8>(ext, lane));
+    ext = __builtin_amdgcn_readfirstlane(ext);
+    const uint32_t kmx = ext & 0xFFFFu, kmn = 0xFFFFu - (ext >> 16);
+    // A NaN (above +inf's key or below -inf's), a +inf, nothing above -inf, or
+    // x = logit / t past the largest float: the other paths. (uniform)
+    if (kmx >= Inf16<T>::kPosKey || kmn < Inf16<T>::kNegKey || kmx <= Inf16<T>::kNegKey) return -1;
+    auto value = [](uint32_t key) { return lo_f<T>(key_bits(key)); };
+    const float top = value(kmx), kcv = 1.4426950408889634f / t;
+    if (!(fabsf(__fdiv_rn(top, t)) < INFINITY)) return -1;
+    // The last bin that may weigh something: 41 binary orders below the
+    // maximum, and two keys more. (-inf's key is never one.)
+    uint32_t klo = pk_key(from_float<T>(top - 41.f / kcv).x) & 0xFFFFu;
+    klo = max(klo, Inf16<T>::kNegKey + 3u) - 2u;
+    const uint32_t span = __builtin_amdgcn_readfirstlane(kmx - klo);
+    if (span >= static_cast<uint32_t>(kKeyBins)) return -1;
+    // 2.
+    const uint32_t top2 = kmx * 0x10001u;
+    auto count_chunk = [&](const u32x4& w) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t x = __builtin_bit_cast(
+            uint32_t, __builtin_bit_cast(u16x2, top2) - __builtin_bit_cast(u16x2, static_cast<uint32_t>(w[e])));
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+          const uint32_t bin = y ? x >> 16 : x & 0xFFFFu;
+          if (bin <= span) atomicAdd(&q.bins[bin], 1u);
+        }
+      }
+    };
+#pragma unroll
+    for (int j = 0; j < kRegChunks; ++j) {
+      if ((j + 1) * kSampThreads <= n8) {  // (uniform)
+        count_chunk(ch[j]);
+      } else if (tid + j * kSampThreads < n8) {
+        count_chunk(ch[j]);
+      }
+    }
+    __syncthreads();
+    // 3. The number of elements in a bin: the two zeros rank as one value, +0.
+    const uint32_t zero_bin = kmx >= 0x8000u ? kmx - 0x8000u : 0x20000u;  // +0's (-0's is the next)
+    const uint32_t minus_zeros = zero_bin < span ? q.bins[zero_bin + 1] : 0u;
+    auto bin_count = [&](uint32_t bin) {
+      const uint32_t c = q.bins[bin];
+      return bin == zero_bin ? c + minus_zeros : (bin == zero_bin + 1 ? 0u : c);
+    };
+    auto mass_at = [&](uint32_t bin) { return mass_of(value(kmx - bin), top, kcv); };
+    const int n_blocks = static_cast<int>(span >> 6) + 1;
+    for (int b0 = wave; b0 < n_blocks; b0 += 8 * kSampWaves) {
+      uint32_t cs[8];  // (read together; past the last block: empty)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int b = b0 + i * kSampWaves;
+        cs[i] = b < n_blocks ? bin_count(static_cast<uint32_t>(64 * b + lane)) : 0u;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (!__any(cs[i] != 0)) continue;  // (uniform; most blocks are empty)
+        const int b = b0 + i * kSampWaves;
+        const uint32_t tc = wave_scan_u32(cs[i]);
+        const uint64_t tm = wave_scan_u64(cs[i] * mass_at(static_cast<uint32_t>(64 * b + lane)));
+        if (lane == 63) {
+          q.bcnt[b] = tc;
+          q.bmass[b] = tm;
+        }
+      }
+    }
+    __syncthreads();
+    const uint32_t bc = q.bcnt[tid];
+    const uint64_t bm = q.bmass[tid];
+    uint32_t ic = wave_scan_u32(bc);
+    uint64_t im = wave_scan_u64(bm);
+    if (lane == 63) {
+      q.wave_c[wave] = ic;
+      q.wave_m[wave] = im;
+    }
+    __syncthreads();
+    uint64_t total = 0;
+#pragma unroll
+    for (int w = 0; w < kSampWaves; ++w) {
+      if (w < wave) {
+        ic += q.wave_c[w];
+        im += q.wave_m[w];
+      }
+      total += q.wave_m[w];
+    }
+    // 4. The first element, in rank order, whose running count and mass (it
+    // included) meet a condition that stays met from there on.
+    struct Place {
+      uint32_t rank, key, nth;  // elements through it; its key, and its place among that key's
+      uint64_t mass;            // running mass through it
+    };
+    auto find = [&](int slot, auto met, Place& r) {
+      const bool hit = bc != 0 && met(ic, im) && (ic == bc || !met(ic - bc, im - bm));  // (one thread at most)
+      const uint64_t hits = __ballot(hit);
+      if (hits != 0) {  // (uniform)
+        const int own = __builtin_ctzll(hits);
+        auto lane64 = [](uint64_t x, int src) {
+          return (static_cast<uint64_t>(
+                      static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x >> 32), src)))
+                  << 32) |
+                 static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), src));
+        };
+        const uint32_t before_c = __builtin_amdgcn_readlane(ic - bc, own);
+        const uint64_t before_m = lane64(im - bm, own);
+        const uint32_t bin = static_cast<uint32_t>(64 * (64 * wave + own) + lane);
+        const uint32_t c = bin_count(bin);
+        const uint64_t m = c != 0 ? mass_at(bin) : 0;
+        const uint32_t lc = wave_scan_u32(c) + before_c;
+        const uint64_t lm = wave_scan_u64(c * m) + before_m;
+        const int src = __builtin_ctzll(__ballot(c != 0 && met(lc, lm)) | (uint64_t{1} << 63));
+        const uint32_t cs = __builtin_amdgcn_readlane(c, src), c0 = __builtin_amdgcn_readlane(lc, src) - cs;
+        const uint64_t ms = lane64(m, src), m0 = lane64(lm, src) - cs * ms;
+        // The place among the key's cs elements: 64 probes a step.
+        uint32_t lo = 0, n = cs;  // in (lo, lo + n]
+        while (n > 1) {
+          const uint32_t step = (n + 63) / 64, i = lo + min(n, (lane + 1) * step);
+          const int f = __builtin_ctzll(__ballot(met(c0 + i, m0 + i * ms)) | (uint64_t{1} << 63));
+          const uint32_t before = min(n - 1, f * step);
+          lo += before;
+          n = min(step, n - before);
+        }
+        if (lane == 0) {
+          q.place_m[slot] = m0 + (lo + 1) * ms;
+          q.place_rank[slot] = c0 + lo + 1;
+          q.place_nth[slot] = lo + 1;
+          q.place_key[slot] = kmx - (bin & ~63u) - static_cast<uint32_t>(src);
+        }
+      }
+      __syncthreads();
+      r.rank = __builtin_amdgcn_readfirstlane(q.place_rank[slot]);
+      r.key = __builtin_amdgcn_readfirstlane(q.place_key[slot]);
+      r.nth = __builtin_amdgcn_readfirstlane(q.place_nth[slot]);
+      r.mass = q.place_m[slot];
+      return r.rank != 0;
+    };
+    Place r;
+    uint64_t z = total;
+    uint32_t lim = 0xFFFFFFFFu;
+    if (k > 0 && k < a.V && find(0, [&](uint32_t c, uint64_t) { return static_cast<int64_t>(c) >= k; }, r)) {
+      z = r.mass;
+      lim = r.rank;
+    }
+    // top-p: the first rank whose running mass exceeds p * Z is the last kept
+    uint64_t kept = z;
+    const double tp = p * static_cast<double>(z);
+    if (find(1, [&](uint32_t, uint64_t m) { return static_cast<double>(m) > tp; }, r) && r.rank <= lim) {
+      kept = r.mass;
+      lim = r.rank;
+    }
+    // the pick: the first kept rank whose running mass reaches u * (kept mass)
+    const double tu = u * static_cast<double>(kept);
+    if (!find(2, [&](uint32_t, uint64_t m) { return static_cast<double>(m) >= tu; }, r) || r.rank > lim) return -1;
+    // 5. Elements with the pick's key, per chunk span and wave, in index order.
+    if (r.key == 0x8000u) {  // (uniform) either zero
+#pragma unroll
+      for (int j = 0; j < kRegChunks; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          uint32_t w = ch[j][e];
+          if ((w & 0xFFFFu) == 0x7FFFu) w += 1u;
+          if ((w >> 16) == 0x7FFFu) w += 0x10000u;
+          ch[j][e] = w;
+        }
+    }
+    const uint32_t want = r.key * 0x10001u;
+    // Whether any of a chunk's eight keys is the pick's (packed: a half of
+    // some word's difference is 0), and which.
+    auto has_match = [&](const u32x4& w) __attribute__((always_inline)) {
+      const uint32_t m = pk_min(pk_min(w[0] ^ want, w[1] ^ want), pk_min(w[2] ^ want, w[3] ^ want));
+      return min(m & 0xFFFFu, m >> 16) == 0;
+    };
+    auto matches = [&](const u32x4& w) __attribute__((always_inline)) {
+      uint32_t m8 = 0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        m8 |= (((e & 1) ? w[e >> 1] >> 16 : w[e >> 1] & 0xFFFFu) == r.key ? 1u : 0u) << e;
+      return m8;
+    };
+#pragma unroll
+    for (int j = 0; j < kRegChunks; ++j) {
+      uint32_t n = 0;
+      const bool any = has_match(ch[j]) && tid + j * kSampThreads < n8;
+      if (__any(any)) {  // (uniform)
+        const uint32_t m8 = any ? matches(ch[j]) : 0u, cnt = __popc(m8);
+#pragma unroll
+        for (int bit = 0; bit < 4; ++bit) n += static_cast<uint32_t>(__popcll(__ballot((cnt >> bit) & 1u))) << bit;
+      }
+      if (lane == 0) q.match[j * kSampWaves + wave] = n;
+    }
+    __syncthreads();
+    // One wave finds the cell and the place in it: the owner of the cell,
+    // which every wave can name.
+    constexpr int kCells = kRegChunks * kSampWaves, kCellsPer = (kCells + 63) / 64;
+    uint32_t cell[kCellsPer], mine = 0;
+#pragma unroll
+    for (int i = 0; i < kCellsPer; ++i) {
+      const int x = kCellsPer * lane + i;
+      cell[i] = x < kCells ? q.match[x] : 0u;
+      mine += cell[i];
+    }
+    const uint32_t incl = wave_scan_u32(mine);
+    int at_cell = -1;
+    uint32_t before = incl - mine, left = 0;
+#pragma unroll
+    for (int i = 0; i < kCellsPer; ++i) {
+      if (before < r.nth && before + cell[i] >= r.nth) {
+        at_cell = kCellsPer * lane + i;
+        left = r.nth - before;
+      }
+      before += cell[i];
+    }
+    const uint64_t owner = __ballot(at_cell >= 0);
+    if (owner == 0) return -1;  // (uniform; never expected: the counts are the registers' own)
+    const int src = __builtin_ctzll(owner);
+    const int c_at = __builtin_amdgcn_readlane(at_cell, src);
+    left = __builtin_amdgcn_readlane(left, src);
+    if (wave == c_at % kSampWaves) {
+      const int js = c_at / kSampWaves;
+      u32x4 w = ch[0];
+#pragma unroll
+      for (int j = 1; j < kRegChunks; ++j)
+        if (j == js) w = ch[j];  // (uniform)
+      const uint32_t m8 = tid + js * kSampThreads < n8 ? matches(w) : 0u;
+      const uint32_t n = __popc(m8), upto = wave_scan_u32(n);
+      if (upto >= left && upto - n < left) {
+        uint32_t rest = m8;
+        for (uint32_t x = upto - n + 1; x < left; ++x) rest &= rest - 1;
+        q.token = static_cast<uint32_t>(8 * (tid + js * kSampThreads) + __builtin_ctz(rest));
+      }
+    }
+    __syncthreads();
+    return static_cast<int64_t>(q.token);
+  }
+
   // Candidate keys: (0xFFFF - key) << 32 | index, with -0's key folded into
   // +0's. Ascending order is the stable descending sort's order (larger
   // values first, ties by index), as for rank_key; cand_value gives back the
@@ -1874,28 +2202,52 @@ __global__ __launch_bounds__(kSampThreads) void sample_tokens_kernel(SampleArgs 
   const int64_t r = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (uniform: an SGPR)
-  const float temp = a.temp[r * a.temp_s];
-  RowSampler<T, UNIT> rs{a, s, static_cast<const T*>(a.logits) + r * a.ls0, fmaxf(temp, 1e-5f), 0.f, tid, lane, wave, 0.f, 0.f};
+  RowSampler<T, UNIT> rs{a, s, static_cast<const T*>(a.logits) + r * a.ls0, 1.f, 0.f, tid, lane, wave, 0.f, 0.f};
+
+  // The row's parameters, then (16-bit rows that fit the registers) the row:
+  // loads complete in order, so the parameters' use waits for them alone
+  // while the row arrives. (top_k as its low and high words, with no branch
+  // on its type between the loads.)
+  const float temp = a.temp[r * a.temp_s], pf = a.topp[r * a.topp_s], uf = a.unif[r * a.unif_s];
+  const int wide_k = a.topk_dt == TSA_I64 ? 1 : 0;
+  const int32_t* const k32 = static_cast<const int32_t*>(a.topk) + ((r * a.topk_s) << wide_k);
+  const int32_t k_lo = k32[0], k_hi = k32[wide_k];
+  u32x4 ch[kRegChunks];
+  bool in_regs = false;
+  if constexpr (UNIT && sizeof(T) == 2) {
+    in_regs = a.cand && rs.chunked() && a.V <= kRegMaxV;
+    __builtin_amdgcn_sched_barrier(0);
+    if (in_regs) rs.load_row(ch);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  rs.t = fmaxf(temp, 1e-5f);
+  const int64_t k = wide_k ? static_cast<int64_t>((static_cast<uint64_t>(static_cast<uint32_t>(k_hi)) << 32) |
+                                                  static_cast<uint32_t>(k_lo))
+                           : static_cast<int64_t>(k_lo);
 
   // Split rows: their statistics and histogram were made by
   // sample_split_stats and sample_split_hist.
-  const bool split = split_row(a, temp, load_int(a.topk, a.topk_dt, r * a.topk_s));
+  const bool split = split_row(a, temp, k);
 
-  // Top-k and greedy rows of a 16-bit row that fits the registers: the
-  // candidate pass decides from one read of the row, or sends it on.
+  // The candidate pass (top-k and greedy rows) and the key-count pass decide
+  // from one read of the row, or send it on.
   if constexpr (UNIT && sizeof(T) == 2) {
-    if (!split && a.cand && rs.chunked() && a.V <= kRegMaxV) {
-      // The row's parameters are loaded first: loads complete in order, so
-      // the test below waits for them alone while the row is in flight.
-      const int64_t k = load_int(a.topk, a.topk_dt, r * a.topk_s);
-      const float pf = a.topp[r * a.topp_s], uf = a.unif[r * a.unif_s];
-      u32x4 ch[kRegChunks];
-      rs.load_row(ch);
+    if (in_regs && !split) {
       if (candidate_row(a, temp, k)) {
         const int64_t token = rs.candidates(ch, temp, k, pf, uf);
         if (token >= 0) {
           if (tid == 0) a.out[r * a.out_s] = token;
           return;
+        }
+      }
+      if constexpr (std::is_same<T, bf16_t>::value) {
+        if (temp > 0.f && a.keys) {
+          const int64_t token = rs.by_keys(ch, *reinterpret_cast<KeyLds*>(lds_raw), k, pf, uf);
+          if (token >= 0) {
+            if (tid == 0) a.out[r * a.out_s] = token;
+            return;
+          }
+          __syncthreads();  // (the paths below reuse its LDS)
         }
       }
     }
@@ -1958,20 +2310,18 @@ __global__ __launch_bounds__(kSampThreads) void sample_tokens_kernel(SampleArgs 
       fmn = fminf(fmn, ofm);
       inan = min(inan, __shfl_xor(inan, o, 64));
     }
-    __shared__ float red_mx[kSampWaves], red_mn[kSampWaves], red_fm[kSampWaves];
-    __shared__ int red_imx[kSampWaves], red_imn[kSampWaves], red_nan[kSampWaves];
     if (lane == 0) {
-      red_mx[wave] = mx; red_imx[wave] = imx;
-      red_mn[wave] = mn; red_imn[wave] = imn;
-      red_fm[wave] = fmn;
-      red_nan[wave] = inan;
+      s.red_mx[wave] = mx; s.red_imx[wave] = imx;
+      s.red_mn[wave] = mn; s.red_imn[wave] = imn;
+      s.red_fm[wave] = fmn;
+      s.red_nan[wave] = inan;
     }
     __syncthreads();
     for (int w = 0; w < kSampWaves; ++w) {
-      if (red_mx[w] > mx || (red_mx[w] == mx && red_imx[w] < imx)) { mx = red_mx[w]; imx = red_imx[w]; }
-      if (red_mn[w] < mn || (red_mn[w] == mn && red_imn[w] > imn)) { mn = red_mn[w]; imn = red_imn[w]; }
-      fmn = fminf(fmn, red_fm[w]);
-      inan = min(inan, red_nan[w]);
+      if (s.red_mx[w] > mx || (s.red_mx[w] == mx && s.red_imx[w] < imx)) { mx = s.red_mx[w]; imx = s.red_imx[w]; }
+      if (s.red_mn[w] < mn || (s.red_mn[w] == mn && s.red_imn[w] > imn)) { mn = s.red_mn[w]; imn = s.red_imn[w]; }
+      fmn = fminf(fmn, s.red_fm[w]);
+      inan = min(inan, s.red_nan[w]);
     }
   }
   int64_t* out = a.out + r * a.out_s;
@@ -1999,10 +2349,9 @@ __global__ __launch_bounds__(kSampThreads) void sample_tokens_kernel(SampleArgs 
   const float klo = fminf(fmn, mx);
   rs.xmax = rs.key_to_x(mx);  // division never decreases, so these are x's maximum and finite minimum
   const float lo0 = rs.key_to_x(klo);
-  const int64_t k = load_int(a.topk, a.topk_dt, r * a.topk_s);
   const bool cut_k = k > 0 && k < a.V;
-  const double p = a.topp[r * a.topp_s];
-  const double u = a.unif[r * a.unif_s];
+  const double p = pf;
+  const double u = uf;
   int64_t token;
   if (rs.fast(klo, k, cut_k, p, u, token)) {
     if (tid == 0) *out = token;
@@ -2131,12 +2480,16 @@ int sample_impl(const tsa_view* out, const tsa_view* logits, const tsa_view* tem
   // workspace, and a batch small enough (split_segments).
   const bool rows16 = (logits->dtype == TSA_BF16 || logits->dtype == TSA_F16) && a.ls1 == 1 && (V & 7) == 0 &&
                       (reinterpret_cast<uintptr_t>(logits->data) & 15) == 0 && ((a.ls0 * 2) & 15) == 0;
+  // The key-count pass takes bf16 rows of such sizes whole, in one launch.
+  a.keys = a.cand && rows16 && logits->dtype == TSA_BF16 && V >= kKeysMinV && V <= kRegMaxV ? 1 : 0;
   const int S = workspace != nullptr && rows16 ? split_segments(B, V) : 0;
   if (S > 1) {
     const size_t need = split_bytes(B, V, S);
     TSA_REQUIRE(workspace_bytes >= need, "workspace too small: %zu bytes, need %zu (tsa_sample_tokens_workspace_bytes)",
                 workspace_bytes, need);
     TSA_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, "workspace must be 256-byte aligned");
+  }
+  if (S > 1 && !a.keys) {
     const SplitLayout l = split_layout(B, V, S);
     char* w = static_cast<char*>(workspace);
     a.stat = reinterpret_cast<SplitStat*>(w);
@@ -2157,7 +2510,7 @@ int sample_impl(const tsa_view* out, const tsa_view* logits, const tsa_view* tem
       sample_split_hist<f16_t><<<sgrid, dim3(kSplitThreads), 0, st>>>(a);
     }
   }
-  const size_t lds = sizeof(SampleLds);
+  const size_t lds = a.keys && sizeof(KeyLds) > sizeof(SampleLds) ? sizeof(KeyLds) : sizeof(SampleLds);
   switch (logits->dtype) {
     case TSA_BF16:
       if (a.ls1 == 1) sample_tokens_kernel<bf16_t, true><<<dim3(B), dim3(kSampThreads), lds, st>>>(a);

@@ -2,7 +2,7 @@
 (server/model/sampling.py:119-194), on the gfx950 HIP library.
 
 Same signature, argument meaning and ValueError messages. One launch samples
-every row (three for a small batch of long 16-bit rows, whose statistics and
+every row (three for a small batch of long f16 rows, whose statistics and
 histogram passes are spread over several workgroups per row, through a
 workspace allocated here); nothing synchronises with the host (the caller's
 ``.tolist()`` is the step's one sync, as in the reference). The kernel finds the top-k cut, the
