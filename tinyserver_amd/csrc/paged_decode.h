@@ -24,7 +24,6 @@ struct DecodeArgs {
   int32_t B, Hq, Hkv, G, BS, max_blocks, D;
   int32_t W;        // workgroups of the stream kernel
   int32_t NW;       // wave workers sharing the tile list (kWaves * W)
-  int32_t unit;     // 1: one workgroup per (sequence, kv head) unit, W = B * Hkv, no merge launch
   float scale_log2;
   float* part;      // [B * Hkv + NW][G * (D + 2)]: per (unit, worker) acc[G][D], m[G], l[G]
   int32_t* pref_out;  // [B + 1] tile prefix over the sequences, for the merge
@@ -35,7 +34,9 @@ struct DecodeArgs {
   void* kc_out; void* vc_out;  // the caches, written (the new token's rows)
   int64_t kn_ss, kn_sh, vn_ss, vn_sh, cs_ss, sn_ss;
   float eps;
-  int32_t S;        // float32 (paged_decode_f32.hip): the splits of a unit's tiles (0: the generic kernel)
+  // Splits of a unit's tiles, in the unit form (16-bit, paged_decode_unit.h; 0:
+  // the stream) and in float32 (paged_decode_f32.hip; 0: the generic kernel).
+  int32_t S;
 };
 
 constexpr float kNegInf = -INFINITY;
@@ -45,6 +46,23 @@ __device__ __forceinline__ int64_t clamp_len(const DecodeArgs& a, int s) {
   int64_t L = a.seq_lens[s * a.sl_s];
   const int64_t cap = static_cast<int64_t>(a.max_blocks) * a.BS;
   return L < 0 ? 0 : (L > cap ? cap : L);
+}
+
+// A 16-byte load, non-temporal (the streaming hint) with NT.
+template <bool NT, typename T>
+__device__ __forceinline__ u32x4 load_stream(const T* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+  else return *reinterpret_cast<const u32x4*>(p);
+}
+
+// Online log-sum-exp: (m, l, o) of more tokens into (M, L, O). A part whose
+// tokens all score -inf has m = -inf and weighs 0 (a NaN in it stays one).
+__device__ __forceinline__ void combine_partial(float& M, float& L, float& O, float m, float l, float o) {
+  const float mn = fmaxf(M, m), mu = mn == kNegInf ? 0.f : mn;
+  const float c_old = fast_exp2(M - mu), c_new = fast_exp2(m - mu);
+  O = fmaf(o, c_new, O * c_old);
+  L = fmaf(l, c_new, L * c_old);
+  M = mn;
 }
 
 // paged_decode_f32.hip: the splits of a unit, whether it takes a float32 call

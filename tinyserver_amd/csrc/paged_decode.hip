@@ -47,10 +47,9 @@
 // * A second kernel merges, per unit, the partials of the wave workers whose
 //   runs cover it with a log-sum-exp reduce. The kernel boundary orders the
 //   two, so no cache flushes or atomics are needed; no host sync, no memset.
-// * Small batches (at most 64 units, tables of at most 512 tokens, no grid
-//   asked for) run one workgroup per unit instead: its four waves split the
-//   unit's tiles through the same ring, leave their partials in LDS, and
-//   the workgroup merges them and writes the output. One launch.
+// * Batches of small block tables take the unit form instead
+//   (paged_decode_unit.h): one workgroup per 512 tokens of a unit, with no
+//   prefix, and no merge launch where a unit has one workgroup.
 //
 // Tokens past seq_len are scored -inf and their V rows zeroed (the
 // reference's masked loads, :88-105). seq_len is clamped to the block table's
@@ -69,6 +68,7 @@
 #include "tsa_common.h"
 #include "norm_rope_row.h"
 #include "paged_decode.h"
+#include "paged_decode_unit.h"
 #include "varlen_prefill_gqa.h"
 
 namespace tsa {
@@ -176,12 +176,6 @@ constexpr int kStreamNtMin = TSA_DECODE_NT_MIN_TILES;
 #define TSA_FUSED_NT_MIN_TILES 128
 #endif
 constexpr int kFusedNtMin = TSA_FUSED_NT_MIN_TILES;
-template <bool NT, typename T>
-__device__ __forceinline__ u32x4 load_stream(const T* p) {
-  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-  else return *reinterpret_cast<const u32x4*>(p);
-}
-
 __device__ __forceinline__ int tiles_of(const DecodeArgs& a, int s) {
   return static_cast<int>((clamp_len(a, s) + 15) >> 4);
 }
@@ -215,59 +209,6 @@ __device__ void tile_prefix_wave(const DecodeArgs& a, int* pref) {
 
 // Position of one wave in the global tile list (unit-major): unit (s, kvh),
 // tile t of the unit's n tiles. Wave-uniform; empty sequences are skipped.
-// One workgroup per unit: the four waves' partials (acc[G][D], m[G], l[G],
-// padded to 16 bytes) in LDS after the tile prefixes -- or, in the fused
-// step, at the start of each wave's own area, which its stream no longer
-// reads once the partial is written (no LDS DMA is in flight by then: the
-// only one, the unit's, lands before the wave's first tile is computed).
-__host__ __device__ inline int unit_slot_floats(int G, int D) { return (G * (D + 2) + 3) & ~3; }
-__host__ __device__ inline int prefix_lds_bytes16(int B) { return (kWaves * (B + 1) * 4 + 15) & ~15; }
-static_assert(kFusedWaveBytes >= 8 * (128 + 2) * 4, "a fused wave's area holds its partial (G <= 8, head_dim 128)");
-template <bool FUSED>
-__device__ __forceinline__ float* unit_slot(const DecodeArgs& a, int* lds_i, int w) {
-  char* const base = reinterpret_cast<char*>(lds_i) + prefix_lds_bytes16(a.B);
-  if constexpr (FUSED) return reinterpret_cast<float*>(base + w * kFusedWaveBytes);
-  else return reinterpret_cast<float*>(base) + w * unit_slot_floats(a.G, a.D);
-}
-
-// Workgroup barrier over the LDS partials only. The fences order LDS and not
-// global memory, so the barrier does not wait for the ring's last loads
-// (repeats of the wave's last tile, whose registers nothing reads).
-__device__ __forceinline__ void unit_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// The merge of one unit's wave partials (after the workgroup barrier):
-// output (head h, dim d) combines the waves that had tiles in wave order,
-// with the running-max rescale of paged_decode_stream_merge. A unit with no
-// tiles (seq_len 0) gives 0/0 = NaN, as the reference's does.
-template <typename T, bool FUSED>
-__device__ __forceinline__ void unit_merge(const DecodeArgs& a, int* lds_i) {
-  const int Hkv = a.Hkv, G = a.G, D = a.D;
-  const int s = blockIdx.x / Hkv, kvh = blockIdx.x - s * Hkv;
-  const int n = lds_i[s + 1] - lds_i[s];  // wave 0's prefix copy
-  const int q = (n + kWaves - 1) / kWaves;
-  const int nw = n == 0 ? 0 : (n + q - 1) / q;
-  T* orow = static_cast<T*>(a.out) + s * a.o_ss + (kvh * G) * a.o_sh;
-  for (int idx = threadIdx.x; idx < G * D; idx += kThreads) {
-    const int hd = idx / D;
-    float M = kNegInf, den = 0.f, o = 0.f;
-    for (int w = 0; w < nw; ++w) {
-      const float* sl = unit_slot<FUSED>(a, lds_i, w);
-      const float mb = sl[G * D + hd], lb = sl[G * D + G + hd], ab = sl[idx];
-      const float mn = fmaxf(M, mb);
-      if (mn == kNegInf) continue;
-      const float c_old = fast_exp2(M - mn), c_new = fast_exp2(mb - mn);
-      o = o * c_old + ab * c_new;
-      den = den * c_old + lb * c_new;
-      M = mn;
-    }
-    orow[hd * a.o_sh + (idx - hd * D) * a.o_sd] = from_float<T>(o / den);
-  }
-}
-
 struct TileCursor {
   int s, kvh, n, t;
   // Values read from the LDS prefix go through readfirstlane, so the compiler
@@ -306,12 +247,11 @@ struct TileCursor {
 // (batches whose prefixes would not fit in LDS) the waves read the tile
 // prefix that decode_tile_prefix wrote to the workspace instead, and the
 // workgroup takes no LDS.
-template <typename T, int D, bool PAGE16, bool CONTIG, bool FUSED, bool GPREF = false, bool UNIT = false>
+template <typename T, int D, bool PAGE16, bool CONTIG, bool FUSED, bool GPREF = false>
 __device__ __forceinline__ void decode_stream_body(DecodeArgs a, const int32_t* __restrict__ bt,
                                                    const int32_t* __restrict__ sl, float* __restrict__ part,
                                                    int* lds_i) {
   static_assert(!(GPREF && FUSED), "the fused step keeps its tile prefixes in LDS");
-  static_assert(!(GPREF && UNIT), "one workgroup per unit keeps its tile prefixes in LDS");
   constexpr int KJ = D / 32;  // k-steps of the score MFMA
   a.bt = bt;
   a.seq_lens = sl;
@@ -321,16 +261,6 @@ __device__ __forceinline__ void decode_stream_body(DecodeArgs a, const int32_t* 
   // Wave-uniform (scalar) so tile indices, block-table reads and page bases
   // stay in SGPRs and the table lookups are scalar loads.
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // One workgroup per unit, 16-token pages: lane i holds the unit's block-table
-  // entry i, loaded beside the sequence lengths, and each tile's page id is a
-  // lane read rather than a dependent scalar load. (The plan takes this form
-  // only for tables of at most kUnitMaxTiles = 32 tiles per unit, so 16-token
-  // or larger pages give at most 32 entries, within the wave's 64 lanes.)
-  int btv = 0;
-  if constexpr (UNIT && PAGE16) {
-    const int us = blockIdx.x / Hkv;
-    if (lane < a.max_blocks) btv = bt[us * a.bt_s0 + lane * a.bt_s1];
-  }
   const int* pref;
   if constexpr (GPREF) {
     pref = a.pref_out;  // [B + 1], written by decode_tile_prefix before this launch
@@ -356,25 +286,10 @@ __device__ __forceinline__ void decode_stream_body(DecodeArgs a, const int32_t* 
   };
 
   const int v = blockIdx.x * kWaves + wave;
-  int64_t lo, hi;
-  if constexpr (UNIT) {
-    // Workgroup u takes unit (u / Hkv, u % Hkv); wave w its w-th quarter
-    // of the unit's n tiles (ceil(n / kWaves) each, the last waves fewer or
-    // none). The wave's partial goes to LDS and the workgroup merges.
-    const int us = blockIdx.x / Hkv, ukvh = blockIdx.x - us * Hkv;
-    const int n = __builtin_amdgcn_readfirstlane(pref[us + 1] - pref[us]);
-    const int q = (n + kWaves - 1) / kWaves;
-    const int64_t u0 = static_cast<int64_t>(Hkv) * __builtin_amdgcn_readfirstlane(pref[us]) +
-                       static_cast<int64_t>(ukvh) * n;
-    lo = u0 + min(n, wave * q);
-    hi = u0 + min(n, (wave + 1) * q);
-  } else {
-    const int64_t total = static_cast<int64_t>(Hkv) * pref[a.B];
-    const int64_t share = (total + a.NW - 1) / a.NW;
-    lo = static_cast<int64_t>(v) * share;
-    hi = min(total, lo + share);
-  }
-  if (lo >= hi) return;  // no barrier follows (one workgroup per unit: the caller's barrier)
+  const int64_t total = static_cast<int64_t>(Hkv) * pref[a.B];
+  const int64_t share = (total + a.NW - 1) / a.NW;
+  const int64_t lo = static_cast<int64_t>(v) * share, hi = min(total, lo + share);
+  if (lo >= hi) return;  // no barrier follows
   const int n_tiles = static_cast<int>(hi - lo);
   if constexpr (FUSED) {  // weights: lanes 0-15 q_weight, 16-31 k_weight (32-63 repeat them)
     const T* wsrc = static_cast<const T*>((lane & 16) ? a.kw : a.qw) + 8 * (lane & 15);
@@ -429,18 +344,6 @@ __device__ __forceinline__ void decode_stream_body(DecodeArgs a, const int32_t* 
     slot = tok - lb * a.BS;
     return phys >= 0 && phys < a.NB;
   };
-  // The page of a tile's first token (tok wave-uniform).
-  auto tile_page = [&](const int32_t* bt_row, int64_t tok, int64_t& phys, int64_t& slot) -> bool {
-    if constexpr (UNIT && PAGE16) {
-      const int lb = static_cast<int>(tok / a.BS);
-      phys = __builtin_amdgcn_readlane(btv, lb);
-      slot = tok - static_cast<int64_t>(lb) * a.BS;
-      return phys >= 0 && phys < a.NB;
-    } else {
-      return page_of(bt_row, tok, phys, slot);
-    }
-  };
-
   // One tile's operands: Q^T (lane (g, c): head c, dims 8(g + 4j)..+8), the K
   // operand (token c of the tile, same dims) and V rows (tokens 4g..4g+3).
   // With 16-token pages the loads are unconditional (an invalid page id reads
@@ -464,7 +367,7 @@ __device__ __forceinline__ void decode_stream_body(DecodeArgs a, const int32_t* 
     const int64_t tok0 = static_cast<int64_t>(tc.t) * 16;
     if constexpr (PAGE16) {
       int64_t phys, slot0;
-      if (!tile_page(bt_row, tok0, phys, slot0)) phys = 0;
+      if (!page_of(bt_row, tok0, phys, slot0)) phys = 0;
       const T* kp = kbase + phys * a.kc_b + (slot0 + c) * ks + 8 * g;
 #pragma unroll
       for (int j = 0; j < KJ; ++j) ko[j] = load_stream<NT>(kp + 32 * j);
@@ -505,7 +408,7 @@ __device__ __forceinline__ void decode_stream_body(DecodeArgs a, const int32_t* 
     int64_t lim = tc.t + 1 < tc.n ? tok0 + 16 : clamp_len(a, tc.s);
     if constexpr (PAGE16) {
       int64_t phys, slot0;
-      if (!tile_page(a.bt + tc.s * a.bt_s0, tok0, phys, slot0)) lim = tok0;
+      if (!page_of(a.bt + tc.s * a.bt_s0, tok0, phys, slot0)) lim = tok0;
     }
     if (tok0 + 16 > lim) {
 #pragma unroll
@@ -576,9 +479,7 @@ __device__ __forceinline__ void decode_stream_body(DecodeArgs a, const int32_t* 
     float lt = l;
     lt += __shfl_xor(lt, 16, 64);
     lt += __shfl_xor(lt, 32, 64);
-    float* slot;
-    if constexpr (UNIT) slot = unit_slot<FUSED>(a, lds_i, wave);
-    else slot = a.part + (static_cast<int64_t>(tc.s) * Hkv + tc.kvh + v) * slot_floats;
+    float* const slot = a.part + (static_cast<int64_t>(tc.s) * Hkv + tc.kvh + v) * slot_floats;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int hd = 4 * g + r;
@@ -727,23 +628,25 @@ __device__ __forceinline__ void decode_stream_body(DecodeArgs a, const int32_t* 
       }
     }
   };
-  // One workgroup per unit (small batches) streams with ordinary loads: the
-  // ring's repeats of the wave's last tile then hit L2 rather than HBM, and
-  // the merge's registers wait for them.
-  if (!UNIT && n_tiles >= (FUSED ? kFusedNtMin : kStreamNtMin)) stream(std::true_type{});
+  if (n_tiles >= (FUSED ? kFusedNtMin : kStreamNtMin)) stream(std::true_type{});
   else stream(std::false_type{});
 }
 
-template <typename T, int D, bool PAGE16, bool CONTIG, bool FUSED, bool GPREF, bool UNIT = false>
+template <typename T, int D, bool PAGE16, bool CONTIG, bool FUSED, bool GPREF>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(TSA_DECODE_WAVES_PER_EU)))
 void paged_decode_stream(DecodeArgs a, const int32_t* __restrict__ bt, const int32_t* __restrict__ sl,
                          float* __restrict__ part) {
   extern __shared__ int lds_i[];
-  decode_stream_body<T, D, PAGE16, CONTIG, FUSED, GPREF, UNIT>(a, bt, sl, part, lds_i);
-  if constexpr (UNIT) {
-    unit_barrier();
-    unit_merge<T, FUSED>(a, lds_i);
-  }
+  decode_stream_body<T, D, PAGE16, CONTIG, FUSED, GPREF>(a, bt, sl, part, lds_i);
+}
+
+// The unit form: grid units x S, NW waves (paged_decode_unit.h).
+template <typename T, int D, bool PAGE16, bool CONTIG, bool FUSED, int NW, bool NT>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void paged_decode_unit(
+    DecodeArgs a, const int32_t* __restrict__ bt, const int32_t* __restrict__ sl, float* __restrict__ part) {
+  extern __shared__ int lds_i[];
+  decode_unit_body<T, D, PAGE16, CONTIG, FUSED, NW, NW, NT>(a, bt, sl, part, blockIdx.x, blockIdx.y,
+                                                       reinterpret_cast<char*>(lds_i));
 }
 
 // The exclusive tile prefix over the sequences (pref_out[0..B], pref_out[B]
@@ -939,7 +842,8 @@ static int default_workgroups() {
 
 struct DecodePlan {
   int W;
-  bool unit;
+  int S;          // splits of a unit in the unit form (0: the stream)
+  int64_t slots;  // partials the workspace holds
   size_t part_bytes, pref_bytes, total;
 };
 
@@ -953,17 +857,25 @@ struct DecodePlan {
 // (Qwen3-0.6B batch of 4, 1024-tile tables: 11.5 us replayed at 128
 // workgroups against 12.6 at 256; a 56-tile batch 10.7 us at any grid).
 constexpr int kMinAutoWG = 64;
-// With no grid asked for, a batch of at most kUnitMaxUnits (sequence, kv
-// head) units whose block tables hold at most kUnitMaxTiles tiles per unit
-// takes one workgroup per unit instead: its four waves split the unit's
-// tiles, merge in LDS and write the output, so the call is one launch with
-// no merge launch after it. Its waves compute their tiles one after
-// another (about 0.7 us of computation per tile, measured), so it pays only
-// while the units are few and short: the Qwen3-0.6B batch of 4 (32 units,
-// 32-tile tables) went from 11.7 to 10.3-10.5 us replayed.
-constexpr int64_t kUnitMaxUnits = 64;
-constexpr int64_t kUnitMaxTiles = 32;
-static_assert(kUnitMaxTiles <= 64, "a unit's block-table row (16-token or larger pages) fits one wave's lanes");
+// With no grid asked for, a batch whose units hold few tiles takes the unit
+// form (paged_decode_unit.h): one workgroup a unit for tables of at most 32
+// tiles, else one per 16 tiles. The limits, in workgroups, lie where the stream
+// takes over (unit form / stream + merge, us a call, K/V rotating over three
+// caches; ctx: tokens a sequence):
+//   one a unit (kUnitMaxUnits):   64 x 64-512 ctx (512 units) 19.1 / 23.8, 90 x
+//     64-512 (720) 26.8 / 27.9, 120 x 64-512 (960) 39.9 / 37.5
+//   split (kUnitMaxWG):   8 x 256-4096 (1,024) 19.1 / 24.1, 16 x 128-2048 fused
+//     (1,024) 27.3 / 31.5, 64 x 64-1024 (2,048) 36.7 / 32.5
+//   long units (kNtSplits; kLongMaxWG): 1 x 20,000-32,768 (1,024) 29.5 / 47, 8 x
+//     8,192 (2,048) 49 / 54, 2 x 32,768 (2,048) 51 / 59
+// The split form's partials must fit kUnitMaxPartBytes, inside what the
+// no-allocation scratch holds. A single workgroup a unit of at most
+// kUnitNoSlots units needs no slots in the workspace.
+constexpr int64_t kUnitMaxUnits = 768;
+constexpr int64_t kUnitMaxWG = 1024;
+constexpr int64_t kLongMaxWG = 2048;
+constexpr int64_t kUnitNoSlots = 64;
+constexpr int64_t kUnitMaxPartBytes = int64_t{15} << 20;
 static DecodePlan make_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t max_blocks, int64_t BS,
                             int32_t num_workgroups) {
   DecodePlan p{};
@@ -975,14 +887,19 @@ static DecodePlan make_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64
     const int64_t cap_tiles = Hkv * B * unit_tiles;
     const int64_t want = (cap_tiles + 2 * kWaves - 1) / (2 * kWaves);
     if (want < p.W) p.W = static_cast<int>(want < kMinAutoWG ? kMinAutoWG : want);
-    if (B > 0 && B * Hkv <= kUnitMaxUnits && unit_tiles <= kUnitMaxTiles) {
-      p.unit = true;
-      p.W = static_cast<int>(B * Hkv);
-    }
+    // (one workgroup of kUnitWaves waves, or splits of kSplitWaves)
+    const int64_t units = B * Hkv, split_tiles = kSplitWaves * kWaveTiles;
+    const int64_t splits = unit_tiles <= kUnitWaves * kWaveTiles ? 1 : (unit_tiles + split_tiles - 1) / split_tiles;
+    const int64_t limit = splits == 1 ? kUnitMaxUnits : splits < kNtSplits ? kUnitMaxWG : kLongMaxWG;
+    if (units > 0 && units * splits <= limit &&
+        (splits == 1 || units * splits * (Hq / Hkv) * (D + 2) * 4 <= kUnitMaxPartBytes))
+      p.S = static_cast<int>(splits);
   }
   const int64_t G = Hq / Hkv;
-  // (one workgroup per unit keeps its partials in LDS: no slots)
-  const int64_t slots = p.unit ? 0 : B * Hkv + static_cast<int64_t>(kWaves) * p.W;
+  const bool no_slots = p.S == 1 && B * Hkv <= kUnitNoSlots;
+  int64_t slots = no_slots ? 0 : B * Hkv + static_cast<int64_t>(kWaves) * p.W;
+  if (p.S > 1 && B * Hkv * p.S > slots) slots = B * Hkv * p.S;
+  p.slots = slots;
   p.part_bytes = align256(static_cast<size_t>(slots) * G * (D + 2) * sizeof(float));
   p.pref_bytes = align256(static_cast<size_t>(B + 1) * sizeof(int32_t));
   p.total = p.part_bytes + p.pref_bytes;
@@ -998,6 +915,14 @@ static int launch_merge(const DecodeArgs& a, hipStream_t stream) {
   else if (outs <= 2) paged_decode_stream_merge<T, 2><<<mgrid, dim3(256), 0, stream>>>(a);
   else if (outs <= 4) paged_decode_stream_merge<T, 4><<<mgrid, dim3(256), 0, stream>>>(a);
   else paged_decode_stream_merge<T, 8><<<mgrid, dim3(256), 0, stream>>>(a);
+  return check_launch("tsa_paged_decode");
+}
+
+// The merge of the unit form's partials, if units were split.
+template <typename T>
+static int launch_split_merge(const DecodeArgs& a, hipStream_t stream) {
+  if (a.S <= 1) return TSA_OK;
+  decode_split_merge<T><<<dim3(a.B * a.Hkv, (a.G * a.D + 63) / 64), dim3(256), 0, stream>>>(a);
   return check_launch("tsa_paged_decode");
 }
 
@@ -1027,27 +952,32 @@ static int launch_decode(DecodeArgs& a, bool mfma, hipStream_t stream, bool fuse
     const bool page16 = a.BS % 16 == 0;
     const bool contig = a.kc_s == a.D && a.vc_s == a.D;
     const dim3 grid(a.W);
-    if (a.unit) {  // one workgroup per unit (the plan keeps such batches' prefixes in LDS), no merge launch
+    if (a.S > 0) {  // the unit form
+      const dim3 ugrid(a.B * a.Hkv, a.S);
+      const int lds_u = unit_lds_bytes(a.G, a.D, fused);
+#define TSA_UNIT_LAUNCH_AS(DD, P16, CT, FU, NW, NT)                                                                  \
+  paged_decode_unit<T, DD, P16, CT, FU, NW, NT><<<ugrid, dim3(64 * NW), lds_u, stream>>>(a, a.bt, a.seq_lens, a.part)
+#define TSA_UNIT_LAUNCH(DD, P16, CT, FU)                                               \
+  do {                                                                                 \
+    if (a.S == 1) TSA_UNIT_LAUNCH_AS(DD, P16, CT, FU, kUnitWaves, false);              \
+    else if (a.S < kNtSplits) TSA_UNIT_LAUNCH_AS(DD, P16, CT, FU, kSplitWaves, false); \
+    else TSA_UNIT_LAUNCH_AS(DD, P16, CT, FU, kSplitWaves, true);                       \
+  } while (0)
       if (fused) {
-        paged_decode_stream<T, 128, true, true, true, false, true><<<grid, dim3(kThreads), fused_lds_bytes(a.B),
-                                                                    stream>>>(a, a.bt, a.seq_lens, a.part);
-        return check_launch("tsa_paged_decode");
-      }
-      const size_t lds_u = prefix_lds_bytes16(a.B) + static_cast<size_t>(kWaves) * unit_slot_floats(a.G, a.D) * 4;
-#define TSA_UNIT_LAUNCH(DD, P16, CT)                                                                       \
-  paged_decode_stream<T, DD, P16, CT, false, false, true><<<grid, dim3(kThreads), lds_u, stream>>>(a, a.bt, \
-                                                                                             a.seq_lens, a.part)
-      if (a.D == 128) {
-        if (page16 && contig) TSA_UNIT_LAUNCH(128, true, true);
-        else if (page16) TSA_UNIT_LAUNCH(128, true, false);
-        else TSA_UNIT_LAUNCH(128, false, false);
+        TSA_UNIT_LAUNCH(128, true, true, true);
+      } else if (a.D == 128) {
+        if (page16 && contig) TSA_UNIT_LAUNCH(128, true, true, false);
+        else if (page16) TSA_UNIT_LAUNCH(128, true, false, false);
+        else TSA_UNIT_LAUNCH(128, false, false, false);
       } else {
-        if (page16 && contig) TSA_UNIT_LAUNCH(64, true, true);
-        else if (page16) TSA_UNIT_LAUNCH(64, true, false);
-        else TSA_UNIT_LAUNCH(64, false, false);
+        if (page16 && contig) TSA_UNIT_LAUNCH(64, true, true, false);
+        else if (page16) TSA_UNIT_LAUNCH(64, true, false, false);
+        else TSA_UNIT_LAUNCH(64, false, false, false);
       }
 #undef TSA_UNIT_LAUNCH
-      return check_launch("tsa_paged_decode");
+#undef TSA_UNIT_LAUNCH_AS
+      if (int rc = check_launch("tsa_paged_decode")) return rc;
+      return launch_split_merge<T>(a, stream);
     }
     if (gpref) {
       decode_tile_prefix<<<dim3(1), dim3(kPrefixThreads), 0, stream>>>(a);
@@ -1150,7 +1080,7 @@ static int check_decode(const tsa_view* out, const tsa_view* query, const tsa_vi
     plan = make_plan(B, Hq, Hkv, D, block_tables->size[1], BS, num_workgroups);
     a.W = plan.W;
     a.NW = kWaves * plan.W;
-    a.unit = plan.unit ? 1 : 0;
+    a.S = plan.S;
   } else if (dt == TSA_F32 && rows_vec16(query) && rows_vec16(k_cache) && rows_vec16(v_cache) && decode_f32_takes(a)) {
     // The partials of its splits fit the plan's slots, so the workspace the
     // caller was told to bring serves (the one-workgroup-per-unit form has no
@@ -1158,7 +1088,7 @@ static int check_decode(const tsa_view* out, const tsa_view* query, const tsa_vi
     plan = make_plan(B, Hq, Hkv, D, block_tables->size[1], BS, num_workgroups);
     const int64_t units = B * Hkv;
     a.S = units == 0 ? 1 : decode_f32_splits(units, (block_tables->size[1] * BS + 15) / 16,
-                                             plan.unit ? 0 : units + static_cast<int64_t>(kWaves) * plan.W);
+                                             plan.slots);
   }
   return TSA_OK;
 }
@@ -1307,8 +1237,7 @@ constexpr int kMixedLds = gqa_smem_bytes<128, 4>();
 constexpr int64_t kMixedAutoMaxTokens = 512;
 constexpr int64_t kMixedAutoMaxDecodeTokens = 131072;
 static_assert(kMixedLds >= 64 * 1024, "the mixed kernel's LDS also holds the decode tile prefixes (at most 64 KB)");
-static_assert(kMixedLds >= kWaves * (kUnitMaxUnits + 1) * 4 + 16 + kWaves * 16 * (128 + 2) * 4,
-              "the mixed kernel's LDS holds a unit-mode decode workgroup's prefixes and wave partials");
+static_assert(kMixedLds >= kUnitWaves * 16 * (128 + 2) * 4, "the mixed kernel's LDS holds a unit workgroup's partials");
 static_assert(kThreads == 64 * 4 && TSA_DECODE_WAVES_PER_EU == 2,
               "the decode and prefill roles share a 4-wave workgroup compiled for two waves per SIMD");
 
@@ -1318,10 +1247,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     PrefillArgs p, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k) {
   __shared__ __align__(16) char lds_m[kMixedLds];
   if (static_cast<int>(blockIdx.x) < d.W) {
-    if (d.unit) {  // one workgroup per decode unit, merged here (as tsa_paged_decode's plan takes it)
-      decode_stream_body<T, 128, true, true, false, false, true>(d, bt, sl, part, reinterpret_cast<int*>(lds_m));
-      unit_barrier();
-      unit_merge<T, false>(d, reinterpret_cast<int*>(lds_m));
+    if (d.S > 0) {  // the unit form (as tsa_paged_decode's plan takes it): W = units x S, four waves
+      const int units = d.B * d.Hkv, sp = static_cast<int>(blockIdx.x) / units;
+      const int u = static_cast<int>(blockIdx.x) - sp * units;
+      if (d.S == 1) decode_unit_body<T, 128, true, true, false, kUnitWaves, 4>(d, bt, sl, part, u, sp, lds_m);
+      else decode_unit_body<T, 128, true, true, false, kSplitWaves, 4>(d, bt, sl, part, u, sp, lds_m);
     } else {
       decode_stream_body<T, 128, true, true, false>(d, bt, sl, part, reinterpret_cast<int*>(lds_m));
     }
@@ -1381,17 +1311,18 @@ extern "C" int tsa_mixed_attention(const tsa_view* prefill_out, const tsa_view* 
     set_error("unsupported dtype");
     return TSA_ERR_UNSUPPORTED;
   }
+  if (a.S > 0) a.W = a.B * a.Hkv * a.S;  // the decode role's workgroups
   const int P = prefill_workgroups > 0 ? prefill_workgroups : device_cus();
   const dim3 grid(a.W + P);
   if (dt == TSA_BF16) {
     mixed_attention_kernel<bf16_t><<<grid, dim3(kThreads), 0, st>>>(a, a.bt, a.seq_lens, a.part, pa, pa.cu_q,
                                                                      pa.cu_k);
     if (int rc = check_launch("tsa_mixed_attention")) return rc;
-    return a.unit ? TSA_OK : launch_merge<bf16_t>(a, st);
+    return a.S > 0 ? launch_split_merge<bf16_t>(a, st) : launch_merge<bf16_t>(a, st);
   }
   mixed_attention_kernel<f16_t><<<grid, dim3(kThreads), 0, st>>>(a, a.bt, a.seq_lens, a.part, pa, pa.cu_q, pa.cu_k);
   if (int rc = check_launch("tsa_mixed_attention")) return rc;
-  return a.unit ? TSA_OK : launch_merge<f16_t>(a, st);
+  return a.S > 0 ? launch_split_merge<f16_t>(a, st) : launch_merge<f16_t>(a, st);
 }
 
 // ---------------------------------------------------------------------------

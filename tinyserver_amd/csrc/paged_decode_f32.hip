@@ -34,16 +34,6 @@ constexpr int kF32Waves = 4;
 // the workspace they are not padded.)
 __host__ __device__ inline int f32_slot_floats(int G, int D) { return (G * (D + 2) + 3) & ~3; }
 
-// Online log-sum-exp: (m, l, o) of more tokens into (M, L, O). A part whose
-// tokens all score -inf has m = -inf and weighs 0 (a NaN in it stays one).
-__device__ __forceinline__ void f32_combine(float& M, float& L, float& O, float m, float l, float o) {
-  const float mn = fmaxf(M, m), mu = mn == kNegInf ? 0.f : mn;
-  const float c_old = fast_exp2(M - mu), c_new = fast_exp2(m - mu);
-  O = fmaf(o, c_new, O * c_old);
-  L = fmaf(l, c_new, L * c_old);
-  M = mn;
-}
-
 // Split sp of unit u, by the whole workgroup: the waves' partials into
 // slots[wave]. (No barrier at the end.)
 template <int D>
@@ -236,14 +226,14 @@ __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
       for (int w = 0; w < kF32Waves; ++w) {
         const float* sl = slots + w * slot;
-        f32_combine(wm, wl, wo, sl[G * D + hd], sl[G * D + G + hd], sl[idx]);
+        combine_partial(wm, wl, wo, sl[G * D + hd], sl[G * D + G + hd], sl[idx]);
       }
       if constexpr (LOOP) {
-        f32_combine(M[k], den[k], o[k], wm, wl, wo);
+        combine_partial(M[k], den[k], o[k], wm, wl, wo);
       } else if (a.S == 1) {
         M[k] = kNegInf;
         den[k] = o[k] = 0.f;
-        f32_combine(M[k], den[k], o[k], wm, wl, wo);
+        combine_partial(M[k], den[k], o[k], wm, wl, wo);
       } else {
         float* const out = a.part + (static_cast<int64_t>(u) * a.S + sp) * (G * (D + 2));
         out[idx] = wo;
@@ -287,7 +277,7 @@ __global__ __launch_bounds__(256) void paged_decode_f32_merge(DecodeArgs a) {
       }
 #pragma unroll
       for (int k = 0; k < 8; ++k)
-        if (sp + k < a.S) f32_combine(M, den, o, pm[k], pl[k], po[k]);
+        if (sp + k < a.S) combine_partial(M, den, o, pm[k], pl[k], po[k]);
     }
     orow[hd * a.o_sh + (idx % D) * a.o_sd] = o / den;
   }
