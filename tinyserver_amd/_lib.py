@@ -1,8 +1,10 @@
-"""ctypes binding of libtsa.so (include/tsa_api.h).
+"""Binding of libtsa.so (include/tsa_api.h).
 
 Tensors cross the boundary as ``tsa_view`` structs (data pointer, sizes,
 element strides, dtype); the HIP stream is torch's current stream on the
-tensor's device. There is no CPU fallback: a missing library raises.
+tensor's device. The compute entry points go through the _tsa_host extension
+(``call``), the others, and tensor subclasses, through ctypes. There is no CPU
+fallback: a missing library raises.
 """
 
 from __future__ import annotations
@@ -98,6 +100,36 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+_host = None
+_entry: dict[str, int] = {}
+
+
+def host():
+    """The _tsa_host extension, loaded once (libtsa.so before it: both are
+    one build). Raises if it has not been built."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _tsa_host
+        except ImportError as e:
+            raise RuntimeError("tinyserver_amd/_tsa_host.so is missing or does not load: build it first "
+                               "(python -m tinyserver_amd._build or __graft_entry__.build())") from e
+        _entry.update({name: i for i, name in enumerate(_tsa_host.entries())})
+        _host = _tsa_host
+    return _host
+
+
+def call(name: str, *args) -> int:
+    """The status of entry point ``name``, called with ``args`` in its order:
+    tensors (or None) for views, floats, and ints (0 for a NULL pointer)."""
+    h = _host or host()
+    rc = h.call(_entry[name], *args)
+    if rc is None:  # a tensor subclass: its own attributes describe it
+        rc = getattr(load(), name)(*(a if isinstance(a, (int, float)) else view(a) for a in args))
+    return rc
+
+
 # One struct.pack per view (the layout of tsa_view; unused entries stay zero)
 # instead of ctypes field sets, which cost microseconds per call.
 _PACK = [struct.Struct("<Q" + "q" * nd + "x" * (8 * (4 - nd)) + "q" * nd + "x" * (8 * (4 - nd)) + "ii")
@@ -134,8 +166,16 @@ def check(rc: int, what: str) -> None:
     raise RuntimeError(f"{what}: {msg} (status {rc})")
 
 
+_DEVICES: dict[int, torch.device] = {}
+
+
 def require_device(*tensors: torch.Tensor) -> torch.device:
     """All tensors must live on one GPU; the kernels have no CPU path."""
+    idx = (_host or host()).device_index(*tensors)
+    if idx >= 0:
+        if idx not in _DEVICES:
+            _DEVICES[idx] = torch.device("cuda", idx)
+        return _DEVICES[idx]
     dev = None
     for t in tensors:
         if t is None:

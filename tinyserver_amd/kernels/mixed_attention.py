@@ -82,20 +82,18 @@ def mixed_attention(
     if out is None:
         out = torch.empty_like(query)
     num_seqs, num_heads, head_dim = query.shape
-    lib = _lib.load()
     stream = _lib.stream_of(dev)
     nbytes = _ws_bytes(dev, num_seqs, num_heads, k_cache.shape[1], head_dim, block_tables.shape[1], k_cache.shape[2],
                        int(num_workgroups))
     ws = _workspace(dev, stream, nbytes)
-    vp = [_lib.view(t) for t in (prefill_out, prefill_q, prefill_k, prefill_v, cu_seqlens)]
-    vd = [_lib.view(t) for t in (out, query, k_cache, v_cache, block_tables, seq_lens)]
-    rc = lib.tsa_mixed_attention(
-        *map(_lib.ref, vp),
+    rc = _lib.call(
+        "tsa_mixed_attention",
+        prefill_out, prefill_q, prefill_k, prefill_v, cu_seqlens,
         int(max_seqlen),
         float(prefill_scale),
-        *map(_lib.ref, vd),
+        out, query, k_cache, v_cache, block_tables, seq_lens,
         1.0 / math.sqrt(head_dim),
-        ws.data_ptr() if ws is not None else None,
+        ws.data_ptr() if ws is not None else 0,
         ws.numel() if ws is not None else 0,
         int(num_workgroups),
         int(prefill_workgroups),

@@ -90,16 +90,15 @@ def paged_attention_forward(
     if out is None:
         out = torch.empty_like(query)
     softmax_scale = 1.0 / math.sqrt(head_dim)
-    lib = _lib.load()
     stream = _lib.stream_of(dev)
     nbytes = _ws_bytes(dev, num_seqs, num_heads, num_kv_heads, head_dim, block_tables.shape[1], k_cache.shape[2],
                        int(num_workgroups))
     ws = _workspace(dev, stream, nbytes)
-    views = [_lib.view(t) for t in (out, query, k_cache, v_cache, block_tables, seq_lens)]
-    rc = lib.tsa_paged_decode(
-        *map(_lib.ref, views),
+    rc = _lib.call(
+        "tsa_paged_decode",
+        out, query, k_cache, v_cache, block_tables, seq_lens,
         softmax_scale,
-        ws.data_ptr() if ws is not None else None,
+        ws.data_ptr() if ws is not None else 0,
         ws.numel() if ws is not None else 0,
         int(num_workgroups),
         stream,
@@ -144,19 +143,17 @@ def paged_decode_step(
     num_kv_heads = k_cache.shape[1]
     if out is None:
         out = torch.empty_like(q)
-    lib = _lib.load()
     stream = _lib.stream_of(dev)
     nbytes = _ws_bytes(dev, num_seqs, num_heads, num_kv_heads, head_dim, block_tables.shape[1], k_cache.shape[2],
                        int(num_workgroups))
     ws = _workspace(dev, stream, nbytes)
-    v8 = [_lib.view(t) for t in (out, q, k, v, q_weight, k_weight, cos, sin)]
-    v4 = [_lib.view(t) for t in (k_cache, v_cache, block_tables, seq_lens)]
-    rc = lib.tsa_paged_decode_step(
-        *map(_lib.ref, v8),
+    rc = _lib.call(
+        "tsa_paged_decode_step",
+        out, q, k, v, q_weight, k_weight, cos, sin,
         float(eps),
-        *map(_lib.ref, v4),
+        k_cache, v_cache, block_tables, seq_lens,
         1.0 / math.sqrt(head_dim),
-        ws.data_ptr() if ws is not None else None,
+        ws.data_ptr() if ws is not None else 0,
         ws.numel() if ws is not None else 0,
         int(num_workgroups),
         stream,

@@ -40,9 +40,8 @@ def qk_norm_rope(q, k, q_weight, k_weight, cos, sin, eps, *, q_out=None, k_out=N
     dev = _lib.require_device(q, k, q_weight, k_weight, cos, sin)
     q_out = torch.empty(q.shape, dtype=q.dtype, device=dev) if q_out is None else q_out
     k_out = torch.empty(k.shape, dtype=k.dtype, device=dev) if k_out is None else k_out
-    lib = _lib.load()
-    views = [_lib.view(t) for t in (q, k, q_out, k_out, q_weight, k_weight, cos, sin)]
-    rc = lib.tsa_qk_norm_rope(*map(_lib.ref, views), float(eps), _lib.stream_of(dev))
+    rc = _lib.call("tsa_qk_norm_rope", q, k, q_out, k_out, q_weight, k_weight, cos, sin, float(eps),
+                   _lib.stream_of(dev))
     _lib.check(rc, "qk_norm_rope")
     return q_out, k_out
 
@@ -62,9 +61,7 @@ def qk_norm_rope_store(
     q_out = torch.empty(q.shape, dtype=q.dtype, device=dev) if q_out is None else q_out
     if return_k and k_out is None:
         k_out = torch.empty(k.shape, dtype=k.dtype, device=dev)
-    lib = _lib.load()
-    views = [_lib.view(t) for t in (q, k, v, q_out, k_out, q_weight, k_weight, cos, sin)]
-    store = [_lib.view(t) for t in (k_cache, v_cache, block_tables, cu_seqlens, positions)]
-    rc = lib.tsa_qk_norm_rope_store(*map(_lib.ref, views), float(eps), *map(_lib.ref, store), _lib.stream_of(dev))
+    rc = _lib.call("tsa_qk_norm_rope_store", q, k, v, q_out, k_out, q_weight, k_weight, cos, sin, float(eps), k_cache,
+                   v_cache, block_tables, cu_seqlens, positions, _lib.stream_of(dev))
     _lib.check(rc, "qk_norm_rope_store")
     return q_out, k_out

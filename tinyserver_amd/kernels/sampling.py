@@ -53,13 +53,13 @@ def sample_tokens(
     if out is None:
         out = torch.empty(batch_size, dtype=torch.int64, device=dev)
     lib = _lib.load()
-    views = [_lib.view(t) for t in (out, logits, temperature, top_k, top_p, uniforms)]
     nbytes = _workspace_bytes(lib, *logits.shape)
     if nbytes:
         ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-        rc = lib.tsa_sample_tokens_ws(*map(_lib.ref, views), ws.data_ptr(), nbytes, _lib.stream_of(dev))
+        rc = _lib.call("tsa_sample_tokens_ws", out, logits, temperature, top_k, top_p, uniforms, ws.data_ptr(), nbytes,
+                       _lib.stream_of(dev))
     else:
-        rc = lib.tsa_sample_tokens(*map(_lib.ref, views), _lib.stream_of(dev))
+        rc = _lib.call("tsa_sample_tokens", out, logits, temperature, top_k, top_p, uniforms, _lib.stream_of(dev))
     _lib.check(rc, "sample_tokens")
     return out
 

@@ -45,10 +45,9 @@ def flash_attn_varlen_func(
         cu_seqlens_k = cu_seqlens_k.to(torch.int32)
     if out is None:
         out = torch.empty_like(q)
-    lib = _lib.load()
-    views = [_lib.view(t) for t in (out, q, k, v, cu_seqlens_q, cu_seqlens_k)]
-    rc = lib.tsa_varlen_prefill(
-        *map(_lib.ref, views),
+    rc = _lib.call(
+        "tsa_varlen_prefill",
+        out, q, k, v, cu_seqlens_q, cu_seqlens_k,
         int(max_seqlen_q),
         int(max_seqlen_k),
         1 if causal else 0,
