@@ -176,11 +176,11 @@ __global__ __launch_bounds__(256) void varlen_prefill_mfma(PrefillArgs a) {
 
 // The standalone LDS-staged GQA kernel (prefill_gqa_body in
 // varlen_prefill_gqa.h): the grid is as many workgroups as fit on the device.
-template <typename T, int D, int NW>
+template <typename T, int D, int NW, int QS>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void varlen_prefill_gqa(
     PrefillArgs a, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k) {
   __shared__ __align__(16) char smem[gqa_smem_bytes<D, NW>()];
-  prefill_gqa_body<T, D, NW>(a, cu_q, cu_k, smem, 0);
+  prefill_gqa_body<T, D, NW, QS>(a, cu_q, cu_k, smem, 0);
 }
 
 // Generic path: one wave per (query row, q-head), fp32 VALU.
@@ -204,12 +204,12 @@ __global__ __launch_bounds__(64) void varlen_prefill_generic(PrefillArgs a, int6
 
 // The persistent kernel runs as many workgroups as fit on the device at once
 // (the occupancy the compiler's resources allow, times the CU count).
-template <typename T, int D, int NW>
+template <typename T, int D, int NW, int QS = 1>
 static int launch_persistent(const PrefillArgs& a, hipStream_t stream) {
   static int per_cu = 0;
   if (per_cu == 0) {
     int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, varlen_prefill_gqa<T, D, NW>, 64 * NW, 0) != hipSuccess || n <= 0)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, varlen_prefill_gqa<T, D, NW, QS>, 64 * NW, 0) != hipSuccess || n <= 0)
       n = 1;
     per_cu = n;
   }
@@ -217,7 +217,7 @@ static int launch_persistent(const PrefillArgs& a, hipStream_t stream) {
   if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       cus <= 0)
     cus = 256;
-  varlen_prefill_gqa<T, D, NW><<<dim3(per_cu * cus), dim3(64 * NW), 0, stream>>>(a, a.cu_q, a.cu_k);
+  varlen_prefill_gqa<T, D, NW, QS><<<dim3(per_cu * cus), dim3(64 * NW), 0, stream>>>(a, a.cu_q, a.cu_k);
   return check_launch("tsa_varlen_prefill");
 }
 
@@ -239,6 +239,8 @@ static bool takes_gqa(const PrefillArgs& a) {
          a.nseq <= max_persist_seqs(a.G) && a.total_q <= int64_t{65535} * 32;
 }
 
+constexpr int64_t kPairMeanLen = 256;
+
 template <typename T>
 static int launch_prefill(PrefillArgs& a, bool mfma, int64_t total_q, int64_t max_seqlen_q, hipStream_t stream) {
   if (a.nseq == 0 || a.Hq == 0 || total_q == 0) return TSA_OK;
@@ -251,6 +253,16 @@ static int launch_prefill(PrefillArgs& a, bool mfma, int64_t total_q, int64_t ma
     if (takes_w64(a)) return prefill_w64_launch(a, sizeof(T) == 2 && std::is_same<T, bf16_t>::value, stream);
     if (takes_gqa(a)) {
       if (a.D == 128) {
+        // Groups of two: four waves take two blocks of 32 queries an item
+        // where sequences average 256 tokens or more -- each K/V block is
+        // staged once for twice the queries, and a CU holds eight waves
+        // instead of six. Shorter sequences leave the second block empty too
+        // often. One block / two, 16/8 heads, us: 8 x 64-960 tokens 31.8 /
+        // 28.9, 4 x 4000-8000 787 / 662, 16 x 500-2000 155 / 136, 3 x 300-900
+        // 20.3 / 20.2; 1 x 200 10.2 / 10.3, 32 x 30-130 15.0 / 16.6. Four
+        // waves of 64 queries (two heads, varlen_prefill_w64's body) took
+        // 35, 649, 142 and 27.9 for the first four.
+        if (a.G == 2 && a.total_q >= kPairMeanLen * a.nseq) return launch_persistent<T, 128, 4, 2>(a, stream);
         if (a.G == 2) return launch_persistent<T, 128, 2>(a, stream);
         if (a.G == 4) return launch_persistent<T, 128, 4>(a, stream);
         return launch_persistent<T, 128, 8>(a, stream);

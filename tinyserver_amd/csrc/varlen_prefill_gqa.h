@@ -94,7 +94,10 @@ constexpr int gqa_smem_bytes() {
 // Scores, probabilities and the output accumulators all stay in VGPRs (at most
 // 256 per wave, two waves per SIMD); the workgroups sharing a CU drift apart,
 // so one workgroup's softmax overlaps another's MFMAs.
-template <typename T, int D, int NW>
+// QS > 1: an item is 32 QS queries, and the workgroup's NW waves take NW / QS
+// q-heads (the group) of QS blocks of 32 queries each, wave w head w % (NW /
+// QS) of block w / (NW / QS).
+template <typename T, int D, int NW, int QS = 1>
 __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* __restrict__ cu_q,
                                                  const int32_t* __restrict__ cu_k, char* smem, int wg_base) {
   constexpr int KJ = D / 16;              // 16-dim steps of the QK reduction
@@ -125,6 +128,8 @@ __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* _
 
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, c = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int HG = NW / QS, IQ = 32 * QS;  // q-heads of the group; queries of an item
+  const int my_head = wave % HG, my_blk = wave / HG;  // this wave's, within the item
   const int nseq = a.nseq, Hkv = a.Hkv;
   const float cs = a.scale_log2;  // > 0 on this path
 
@@ -138,7 +143,7 @@ __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* _
   for (int b = tid; b < nseq; b += 64 * NW) {
     int64_t qs, ql;
     seq_range(cu_q, a.cuq_s, b, a.total_q, qs, ql);
-    nqb_s[b] = static_cast<uint16_t>((ql + 31) / 32);
+    nqb_s[b] = static_cast<uint16_t>((ql + IQ - 1) / IQ);
   }
   __syncthreads();
   // Items above level Q: Hkv * sum_b max(0, nqb_b - Q - 1) (wave reduction).
@@ -158,7 +163,7 @@ __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* _
 
   struct Item {
     int b, kvh, q0, q_len, k_len, nblk;
-    int jm;     // first block that needs a mask (keys past k_len, or causal keys after a query)
+    int jm;     // this wave's first block that needs a mask (keys past k_len, or causal keys after a query)
     int kfull;  // rows below min(k_len, 32 nblk) load without clamping
     int64_t q_start;
     const T* kb;
@@ -197,11 +202,11 @@ __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* _
     it.q_start = qs;
     it.q_len = static_cast<int>(ql);
     it.k_len = static_cast<int>(kl);
-    it.q0 = Q * 32;
-    const int q_last = it.q0 + 32 < it.q_len ? it.q0 + 32 : it.q_len;
+    it.q0 = Q * IQ;
+    const int q_last = it.q0 + IQ < it.q_len ? it.q0 + IQ : it.q_len;
     const int kend = a.causal ? (it.k_len < q_last ? it.k_len : q_last) : it.k_len;
     it.nblk = (kend + 31) / 32;
-    it.jm = a.causal ? min(it.k_len / 32, Q) : it.k_len / 32;
+    it.jm = a.causal ? min(it.k_len / 32, Q * QS + my_blk) : it.k_len / 32;
     it.kfull = min(it.k_len, it.nblk * 32);
     it.kb = static_cast<const T*>(a.k) + ks * a.k_st + it.kvh * a.k_sh;
     it.vb = static_cast<const T*>(a.v) + ks * a.v_st + it.kvh * a.v_sh;
@@ -271,11 +276,11 @@ __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* _
     it.q_start = qs;
     it.q_len = __builtin_amdgcn_readfirstlane(e[3]);
     it.k_len = __builtin_amdgcn_readfirstlane(e[5]);
-    it.q0 = Q * 32;
-    const int q_last = it.q0 + 32 < it.q_len ? it.q0 + 32 : it.q_len;
+    it.q0 = Q * IQ;
+    const int q_last = it.q0 + IQ < it.q_len ? it.q0 + IQ : it.q_len;
     const int kend = a.causal ? (it.k_len < q_last ? it.k_len : q_last) : it.k_len;
     it.nblk = (kend + 31) / 32;
-    it.jm = a.causal ? min(it.k_len / 32, Q) : it.k_len / 32;
+    it.jm = a.causal ? min(it.k_len / 32, Q * QS + my_blk) : it.k_len / 32;
     it.kfull = min(it.k_len, it.nblk * 32);
     it.kb = static_cast<const T*>(a.k) + ks * a.k_st + it.kvh * a.k_sh;
     it.vb = static_cast<const T*>(a.v) + ks * a.v_st + it.kvh * a.v_sh;
@@ -406,8 +411,8 @@ __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* _
   // Q operand of the item (lane (h, c): query q0 + c, dims 16jj + 8h..+8).
   u32x4 qop[KJ];
   auto load_q = [&](const Item& it) {
-    const int row = it.q0 + c;
-    const int head = it.kvh * NW + wave;
+    const int row = it.q0 + 32 * my_blk + c;
+    const int head = it.kvh * HG + my_head;
     const T* qp = static_cast<const T*>(a.q) + (it.q_start + row) * a.q_st + head * a.q_sh;
 #pragma unroll
     for (int jj = 0; jj < KJ; ++jj)
@@ -440,7 +445,7 @@ __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* _
   auto mask_block = [&](const Item& it, f32x16& sc, int blk) {
     const int kb0 = blk * 32;
     if (blk >= it.jm) {
-      const int qq = it.q0 + c;
+      const int qq = it.q0 + 32 * my_blk + c;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int kk = kb0 + 8 * (e >> 2) + 4 * h + (e & 3);
@@ -586,7 +591,7 @@ __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* _
   char* const ost = smem + OOFF + wave * kOutStage;
   auto store_out = [&](const Item& it) {
     const float rl = 1.f / (l + __shfl_xor(l, 32, 64));  // 1 / query c's denominator
-    T* const obase = static_cast<T*>(a.out) + it.q_start * a.o_st + (it.kvh * NW + wave) * a.o_sh;
+    T* const obase = static_cast<T*>(a.out) + it.q_start * a.o_st + (it.kvh * HG + my_head) * a.o_sh;
     const int wsw = (c >> 2) & 3;
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
@@ -603,7 +608,7 @@ __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* _
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const int id = lane + 64 * i, r = id >> 2, q = id & 3;
-        const int row = it.q0 + r;
+        const int row = it.q0 + 32 * my_blk + r;
         const u32x4 w = *reinterpret_cast<const u32x4*>(ost + r * 64 + 16 * (q ^ ((r >> 2) & 3)));
         if (row < it.q_len) *reinterpret_cast<u32x4*>(obase + row * a.o_st + 32 * u + 8 * q) = w;
       }
