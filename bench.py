@@ -265,7 +265,7 @@ def _decode_kernels(w, page, num_workgroups):
     ws = decode_workspace_bytes(B, w.num_heads, w.num_kv_heads, w.q.shape[-1], w.block_tables.shape[1], page,
                                 num_workgroups)
     if ws <= (4 * (B + 1) + 255) // 256 * 256:
-        return "paged_decode_stream (one workgroup per unit, no merge launch)"
+        return "paged_decode_unit (one workgroup per unit, no merge launch)"
     return "paged_decode_stream + paged_decode_stream_merge"
 
 

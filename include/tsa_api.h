@@ -138,8 +138,9 @@ int tsa_qk_norm_rope_store(const tsa_view* q, const tsa_view* k, const tsa_view*
 
 /* Bytes of workspace tsa_paged_decode needs: one partial-result slot per
  * (sequence x kv head, wave) pair that can occur -- num_seqs * num_kv_heads
- * + 4 * num_workgroups slots of (G * head_dim + 2 * G) floats -- and the tile
- * prefix (num_workgroups 0 = the library's choice, one per CU). */
+ * + 4 * num_workgroups slots of (G * head_dim + 2 * G) floats, more where
+ * small tables are split further, none for at most 64 units of one workgroup
+ * -- and the tile prefix (num_workgroups 0 = the library's choice). */
 size_t tsa_paged_decode_workspace_bytes(int64_t num_seqs, int64_t num_heads, int64_t num_kv_heads,
                                         int64_t head_dim, int64_t max_blocks_per_seq,
                                         int64_t block_size, int32_t num_workgroups);
@@ -153,9 +154,11 @@ size_t tsa_paged_decode_workspace_bytes(int64_t num_seqs, int64_t num_heads, int
  * choice: one per CU, fewer for small tables); a second launch merges each
  * sequence's per-wave partial results, which the workspace holds (no
  * initialisation needed; calls that share one must be ordered on one
- * stream). With num_workgroups 0, a batch of at most 64 (sequence, kv head)
- * units whose tables hold at most 512 tokens takes one launch instead: one
- * workgroup per unit, whose waves merge in LDS and write out. Float32 calls
+ * stream). With num_workgroups 0, batches of small block tables take one
+ * workgroup per (sequence, kv head) unit instead, in one launch (up to 768
+ * units whose tables hold at most 512 tokens), or one per 256 tokens of a
+ * unit's table and the merge (up to 1024 of them, 2048 where a table holds
+ * more than 7936 tokens). Float32 calls
  * split each unit over workgroups if the workspace is there, and need none:
  * without it (NULL, or too small) one workgroup computes a unit, with the
  * same result. */

@@ -7,8 +7,9 @@
 // 8192-token sequence of 16/8 heads, 275 GFLOP, runs at 121 here). Small
 // batches are bound by the items' serial parts -- the search, the first loads
 // and the merge, about 7 us a workgroup, of which two share a CU: 8 prompts of
-// 32-512 tokens, 3.5 GFLOP, take 58 us where the products alone need 26.
-// (The one-wave-per-row kernel took 3,355.)
+// 32-512 tokens, 3.5 GFLOP, take 55.5 us where the products alone need 26
+// (57.9 with the sequence's ranges read after the search and K after Q; the
+// one-wave-per-row kernel took 3,355).
 //
 // Work item: 32 rows of one (sequence, kv head), a row being one (query,
 // q-head of the kv head's group), query-major, so one K/V read serves the
@@ -22,7 +23,7 @@
 // score products, the next block's K under the softmax and P V. Blocks of 32
 // keys on the 32x32x2 form took 68 us for that batch (coarser blocks to deal,
 // more masked work); workgroups that stay and walk a precomputed item plan
-// took 59, and 2,430 against 2,264 for the long sequence.
+// took 59 against 58, and 2,430 against 2,264 for the long sequence.
 //
 // Layouts. With lane (g, c) = (lane / 16, lane % 16) and row tiles t = 0, 1:
 //   S^T(16 keys x 16 rows) = K Q^T: step 4 j + i takes dims 16 j + 4 g + i, so
@@ -55,15 +56,23 @@ __device__ __forceinline__ int wave_sum(int x) {
   return __builtin_amdgcn_readlane(static_cast<int>(wave_scan_u32(static_cast<uint32_t>(x))), 63);
 }
 
-// Item j (of the launch's tiles, all kv heads together) -> sequence b, tile t.
+// Item j (of the launch's tiles, all kv heads together) -> its tile t and its
+// sequence's query and key ranges.
 // Up to 64 sequences: latest (heaviest) tiles first over all sequences, by a
 // binary search on the level (the number of tiles at or above a level, summed
 // over the wave's lanes). More sequences: sequence by sequence, latest tile
 // first. Returns false past the last item. Wave-uniform.
-__device__ __forceinline__ bool f32_item(const PrefillArgs& a, int j, int& b, int& t) {
+__device__ __forceinline__ bool f32_item(const PrefillArgs& a, int j, int& t, int64_t& q_start, int64_t& q_len,
+                                         int64_t& k_start, int64_t& k_len) {
   const int lane = threadIdx.x & 63;
+  int b;
   if (a.nseq <= 64) {
-    const int nt = lane < a.nseq ? f32_tiles(a, lane) : 0;
+    // (lane b holds sequence b's ranges: one round trip for all that is read)
+    int64_t qs, ql, ks, kl;
+    const int mine = min(lane, a.nseq - 1);
+    seq_range(a.cu_q, a.cuq_s, mine, a.total_q, qs, ql);
+    seq_range(a.cu_k, a.cuk_s, mine, a.total_k, ks, kl);
+    const int nt = lane < a.nseq ? static_cast<int>((ql * a.G + kF32Rows - 1) / kF32Rows) : 0;
     int mx = nt;
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) mx = max(mx, __shfl_xor(mx, o, 64));
@@ -79,6 +88,11 @@ __device__ __forceinline__ bool f32_item(const PrefillArgs& a, int j, int& b, in
     while (rank-- > 0) mask &= mask - 1;
     b = __builtin_ctzll(mask);
     t = lo;
+    // (starts and lengths fit 31 bits: the host takes calls of fewer rows)
+    q_start = __builtin_amdgcn_readlane(static_cast<int>(qs), b);
+    q_len = __builtin_amdgcn_readlane(static_cast<int>(ql), b);
+    k_start = __builtin_amdgcn_readlane(static_cast<int>(ks), b);
+    k_len = __builtin_amdgcn_readlane(static_cast<int>(kl), b);
     return true;
   }
   const int per = (a.nseq + 63) / 64, b0 = min(a.nseq, lane * per), b1 = min(a.nseq, b0 + per);
@@ -97,6 +111,8 @@ __device__ __forceinline__ bool f32_item(const PrefillArgs& a, int j, int& b, in
   }
   b = __builtin_amdgcn_readfirstlane(b);
   t = __builtin_amdgcn_readfirstlane(nt - 1 - (j - run));
+  seq_range(a.cu_q, a.cuq_s, b, a.total_q, q_start, q_len);
+  seq_range(a.cu_k, a.cuk_s, b, a.total_k, k_start, k_len);
   return true;
 }
 
@@ -119,11 +135,9 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kvh = static_cast<int>(blockIdx.x) % a.Hkv;
-  int b, tile;
-  if (!f32_item(a, static_cast<int>(blockIdx.x) / a.Hkv, b, tile)) return;
+  int tile;
   int64_t q_start, q_len, k_start, k_len;
-  seq_range(a.cu_q, a.cuq_s, b, a.total_q, q_start, q_len);
-  seq_range(a.cu_k, a.cuk_s, b, a.total_k, k_start, k_len);
+  if (!f32_item(a, static_cast<int>(blockIdx.x) / a.Hkv, tile, q_start, q_len, k_start, k_len)) return;
   const int G = a.G;
   // (32-bit rows: the host takes calls of fewer than 2^31 rows)
   const uint32_t row0 = static_cast<uint32_t>(tile) * kF32Rows, n_rows = static_cast<uint32_t>(q_len) * G;
@@ -137,12 +151,16 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
   const int nblk = (kend + 15) / 16;
   const int full = a.causal ? min(kl, q_first + 1) : kl;  // keys below it are seen by every row
 
-  // The item's Q rows into LDS (rows past the last repeat it).
-  for (int i = tid; i < kF32Rows * (D / 4); i += kF32Threads) {
-    const int r = i / (D / 4), ch = i - r * (D / 4);
+  // The item's Q rows (rows past the last repeat it), then the first K block,
+  // all in flight before Q goes to LDS.
+  constexpr int kQ = kF32Rows * (D / 4) / kF32Threads;  // 16-byte pieces a thread
+  f32x4 qv[kQ];
+#pragma unroll
+  for (int x = 0; x < kQ; ++x) {
+    const int i = tid + x * kF32Threads, r = i / (D / 4), ch = i - r * (D / 4);
     const int rr = min(r, rows - 1), qq = q_of(rr);
-    const float* src = static_cast<const float*>(a.q) + (q_start + qq) * a.q_st + head_of(rr, qq) * a.q_sh + 4 * ch;
-    *reinterpret_cast<f32x4*>(smem + r * RP + 4 * ch) = *reinterpret_cast<const f32x4*>(src);
+    qv[x] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(a.q) + (q_start + qq) * a.q_st +
+                                            head_of(rr, qq) * a.q_sh + 4 * ch);
   }
 
   const float* const kb = static_cast<const float*>(a.k) + k_start * a.k_st + kvh * a.k_sh + 4 * g;
@@ -155,6 +173,11 @@ __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(2, 
     for (int j = 0; j < NJ; ++j) kop[j] = *reinterpret_cast<const f32x4*>(p + 16 * j);
   };
   if (wave < nblk) load_k(wave);
+#pragma unroll
+  for (int x = 0; x < kQ; ++x) {
+    const int i = tid + x * kF32Threads, r = i / (D / 4), ch = i - r * (D / 4);
+    *reinterpret_cast<f32x4*>(smem + r * RP + 4 * ch) = qv[x];
+  }
   int my_end[2];  // keys that rows c and 16 + c see
 #pragma unroll
   for (int t = 0; t < 2; ++t) my_end[t] = a.causal ? min(kl, q_of(min(16 * t + c, rows - 1)) + 1) : kl;
