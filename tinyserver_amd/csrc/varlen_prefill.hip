@@ -244,8 +244,8 @@ constexpr int64_t kPairMeanLen = 256;
 template <typename T>
 static int launch_prefill(PrefillArgs& a, bool mfma, int64_t total_q, int64_t max_seqlen_q, hipStream_t stream) {
   if (a.nseq == 0 || a.Hq == 0 || total_q == 0) return TSA_OK;
-  if (!mfma) {
-    if (std::is_same<T, float>::value && a.vec16 && prefill_f32_takes(a)) return prefill_f32_launch(a, stream);
+  if (sizeof(T) == 4 && mfma && prefill_f32_takes(a)) return prefill_f32_launch(a, stream);
+  if (!mfma || sizeof(T) == 4) {
     varlen_prefill_generic<T><<<dim3(total_q, a.Hq), dim3(64), 0, stream>>>(a, total_q);
     return check_launch("tsa_varlen_prefill");
   }
@@ -323,8 +323,7 @@ int prefill_prepare(const tsa_view* out, const tsa_view* q, const tsa_view* k, c
   a.total_q = q->size[0]; a.total_k = k->size[0];
   a.causal = causal ? 1 : 0;
   a.scale_log2 = static_cast<float>(softmax_scale * 1.4426950408889634);
-  a.vec16 = rows_vec16(q) && rows_vec16(k) && rows_vec16(v) && rows_vec16(out) ? 1 : 0;
-  mfma = (dt == TSA_BF16 || dt == TSA_F16) && (D == 64 || D == 128) && a.vec16;
+  mfma = (D == 64 || D == 128) && rows_vec16(q) && rows_vec16(k) && rows_vec16(v) && rows_vec16(out);
   return TSA_OK;
 }
 
@@ -332,7 +331,7 @@ int prefill_launch(PrefillArgs& a, bool mfma, int dtype, int64_t max_seqlen_q, h
   switch (dtype) {
     case TSA_BF16: return launch_prefill<bf16_t>(a, mfma, a.total_q, max_seqlen_q, stream);
     case TSA_F16: return launch_prefill<f16_t>(a, mfma, a.total_q, max_seqlen_q, stream);
-    case TSA_F32: return launch_prefill<float>(a, false, a.total_q, max_seqlen_q, stream);
+    case TSA_F32: return launch_prefill<float>(a, mfma, a.total_q, max_seqlen_q, stream);
   }
   set_error("unsupported dtype");
   return TSA_ERR_UNSUPPORTED;

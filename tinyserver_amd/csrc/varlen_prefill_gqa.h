@@ -25,11 +25,10 @@ struct PrefillArgs {
   int32_t nseq, Hq, Hkv, G, D, nqb;
   int32_t causal;
   float scale_log2;
-  int32_t vec16;  // q, k, v and out rows are unit-stride and 16-byte aligned (host dispatch)
 };
 
-// varlen_prefill_f32.hip: the float32 kernel, and the calls it takes (vec16
-// rows of 64 or 128 dims).
+// varlen_prefill_f32.hip: the float32 kernel, and the calls it takes (of those
+// prefill_prepare marks mfma).
 bool prefill_f32_takes(const PrefillArgs& a);
 int prefill_f32_launch(const PrefillArgs& a, hipStream_t stream);
 
@@ -717,7 +716,8 @@ __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* _
 
 
 // Host side, in varlen_prefill.hip: the checks of tsa_varlen_prefill, filling
-// a (mfma: the 16-bit MFMA kernels may serve the call); the launch of the
+// a (mfma: head_dim 64 or 128 in unit-stride 16-byte aligned rows, which the
+// matrix kernels need); the launch of the
 // kernel it selects; and whether that kernel is varlen_prefill_gqa<T, 128, 4>
 // with these arguments (the one the mixed kernel embeds).
 int prefill_prepare(const tsa_view* out, const tsa_view* q, const tsa_view* k, const tsa_view* v,
