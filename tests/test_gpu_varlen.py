@@ -232,17 +232,18 @@ def test_item_plan_limits_match():
 
 @pytest.mark.parametrize("causal", [True, False])
 def test_groups_of_two_in_pairs(causal):
-    """Two q-heads per kv head: sequences that average 256 tokens or more take
-    items of two 32-query blocks. Block and item edges, q_len != k_len, a
+    """Two q-heads per kv head: sequences that average 384 tokens, enough
+    of them for 352 blocks of 32 queries over the kv heads, take items of two
+    such blocks. Block and item edges, q_len != k_len, a
     sequence without keys; against the oracle, and bit for bit against the
     one-block items the same sequences get beside many short ones."""
-    lq, lk = [1, 31, 32, 33, 63, 64, 65, 97, 128, 40, 2300], [1, 31, 32, 33, 63, 64, 70, 97, 100, 0, 2300]
-    q, k, v, cq, ck = _inputs(lq, lk, 4, 2, 128, torch.bfloat16, seed=51)
+    lq, lk = [1, 31, 32, 33, 63, 64, 65, 97, 128, 40, 3700], [1, 31, 32, 33, 63, 64, 70, 97, 100, 0, 3700]
+    q, k, v, cq, ck = _inputs(lq, lk, 8, 4, 128, torch.bfloat16, seed=51)
     args = [t.to(DEV) for t in (q, k, v)]
     out = flash_attn_varlen_func(*args, cq.to(DEV), ck.to(DEV), max(lq), max(lk), causal).cpu()
-    assert sum(lq) >= 256 * len(lq)
+    assert sum(lq) >= 384 * len(lq) and sum(lq) * 4 >= 352 * 32
     n, t = 300, sum(lq)
-    pad = [x.to(DEV) for x in _inputs([1] * n, [1] * n, 4, 2, 128, torch.bfloat16, seed=52)[:3]]
+    pad = [x.to(DEV) for x in _inputs([1] * n, [1] * n, 8, 4, 128, torch.bfloat16, seed=52)[:3]]
     cq2, ck2 = _cu(lq + [1] * n).to(DEV), _cu(lk + [1] * n).to(DEV)
     one = flash_attn_varlen_func(*(torch.cat(x) for x in zip(args, pad)), cq2, ck2, max(lq), max(lk), causal).cpu()
     ref = ov.flash_attn_varlen_func(q, k, v, cq, ck, max(lq), max(lk), causal)

@@ -239,7 +239,8 @@ static bool takes_gqa(const PrefillArgs& a) {
          a.nseq <= max_persist_seqs(a.G) && a.total_q <= int64_t{65535} * 32;
 }
 
-constexpr int64_t kPairMeanLen = 256;
+constexpr int64_t kPairMeanLen = 384;
+constexpr int64_t kPairItems = 352;
 
 template <typename T>
 static int launch_prefill(PrefillArgs& a, bool mfma, int64_t total_q, int64_t max_seqlen_q, hipStream_t stream) {
@@ -253,16 +254,21 @@ static int launch_prefill(PrefillArgs& a, bool mfma, int64_t total_q, int64_t ma
     if (takes_w64(a)) return prefill_w64_launch(a, sizeof(T) == 2 && std::is_same<T, bf16_t>::value, stream);
     if (takes_gqa(a)) {
       if (a.D == 128) {
-        // Groups of two: four waves take two blocks of 32 queries an item
-        // where sequences average 256 tokens or more -- each K/V block is
-        // staged once for twice the queries, and a CU holds eight waves
-        // instead of six. Shorter sequences leave the second block empty too
-        // often. One block / two, 16/8 heads, us: 8 x 64-960 tokens 31.8 /
-        // 28.9, 4 x 4000-8000 787 / 662, 16 x 500-2000 155 / 136, 3 x 300-900
-        // 20.3 / 20.2; 1 x 200 10.2 / 10.3, 32 x 30-130 15.0 / 16.6. Four
-        // waves of 64 queries (two heads, varlen_prefill_w64's body) took
-        // 35, 649, 142 and 27.9 for the first four.
-        if (a.G == 2 && a.total_q >= kPairMeanLen * a.nseq) return launch_persistent<T, 128, 4, 2>(a, stream);
+        // Groups of two: four waves take two blocks of 32 queries an item --
+        // each K/V block is staged once for twice the queries, and a CU holds
+        // eight waves instead of six. That pays where sequences average 384
+        // tokens (shorter ones leave the second block empty too often) and
+        // one-block items would be at least 352, 1.4 for each CU (fewer run
+        // all at once as they are, and pairs only make each take longer). One
+        // block / two, 16/8 heads, us: 8 x 64-960 tokens 31.8 / 28.9,
+        // 4 x 4000-8000 787 / 662, 16 x 500-2000 155 / 136, 1 x 1500 (376
+        // items) 32.1 / 31.5, 4 x 400 15.1 / 15.2; 1 x 1250 (320) 27.8 / 28.2,
+        // 1 x 569 16.1 / 17.0, 1 x 8000 on one kv head (250) 129 / 132,
+        // 8 x 300 15.4 / 16.2, 16 x 260 20.9 / 23.4. Four waves of 64 queries
+        // (two heads, varlen_prefill_w64's body) took 35, 649 and 142 for the
+        // first three.
+        if (a.G == 2 && a.total_q >= kPairMeanLen * a.nseq && a.total_q * a.Hkv >= kPairItems * 32)
+          return launch_persistent<T, 128, 4, 2>(a, stream);
         if (a.G == 2) return launch_persistent<T, 128, 2>(a, stream);
         if (a.G == 4) return launch_persistent<T, 128, 4>(a, stream);
         return launch_persistent<T, 128, 8>(a, stream);
