@@ -11,6 +11,33 @@ namespace tsa {
 template <typename T>
 __device__ __forceinline__ float round_t(float x) { return to_float(from_float<T>(x)); }
 
+// RoPE's product and sum, each with its own rounding for a 16-bit T. (__fmul_rn
+// and __fadd_rn are plain operators that may contract: in f16 the compiler
+// narrows a product that is rounded to f16 to the f16 multiply and fuses it
+// with the sum, in some kernels and not in others, so that one product is never
+// rounded: 12% of the outputs an ulp away from the model's. Uncontracted, the
+// fused step and the norm/RoPE kernels take the same time (f16, 8 sequences:
+// 21.8 us both ways; 16 packed prompts 71.3 and 71.5). bf16 has no such
+// multiply; in fp32 one rounding fewer is kept.)
+template <typename T>
+__device__ __forceinline__ float rope_mul(float x, float y) {
+  if constexpr (sizeof(T) == 2) {
+#pragma clang fp contract(off)
+    return x * y;
+  } else {
+    return __fmul_rn(x, y);
+  }
+}
+template <typename T>
+__device__ __forceinline__ float rope_add(float x, float y) {
+  if constexpr (sizeof(T) == 2) {
+#pragma clang fp contract(off)
+    return x + y;
+  } else {
+    return __fadd_rn(x, y);
+  }
+}
+
 // Cross-lane moves inside the 16-lane rows of a wave (DPP, no LDS traffic):
 // lane i gets lane i + N of its row (row_shl), or lane (i - N) mod 16
 // (row_ror).
@@ -79,7 +106,7 @@ __device__ __forceinline__ void norm_rope_row(const float (&x)[8], const float (
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const float rot = first_half ? -zp[i] : zp[i];
-    o[i] = round_t<T>(__fadd_rn(round_t<T>(__fmul_rn(z[i], cs[i])), round_t<T>(__fmul_rn(rot, sn[i]))));
+    o[i] = round_t<T>(rope_add<T>(round_t<T>(rope_mul<T>(z[i], cs[i])), round_t<T>(rope_mul<T>(rot, sn[i]))));
   }
 }
 
@@ -155,11 +182,11 @@ __device__ __forceinline__ void norm_rope_row_d128x8(const u32x4 (&xp)[2], const
       const float s0 = lo_f<T>(sp[j][i]), s1 = hi_f<T>(sp[j][i]);
       const float r0 = j == 0 ? -z[1][2 * i] : z[0][2 * i];
       const float r1 = j == 0 ? -z[1][2 * i + 1] : z[0][2 * i + 1];
-      float a0 = __fmul_rn(z[j][2 * i], c0), a1 = __fmul_rn(z[j][2 * i + 1], c1);
+      float a0 = rope_mul<T>(z[j][2 * i], c0), a1 = rope_mul<T>(z[j][2 * i + 1], c1);
       round2_t<T>(a0, a1);
-      float b0 = __fmul_rn(r0, s0), b1 = __fmul_rn(r1, s1);
+      float b0 = rope_mul<T>(r0, s0), b1 = rope_mul<T>(r1, s1);
       round2_t<T>(b0, b1);
-      op[j][i] = pack2<T>(__fadd_rn(a0, b0), __fadd_rn(a1, b1));
+      op[j][i] = pack2<T>(rope_add<T>(a0, b0), rope_add<T>(a1, b1));
     }
 }
 
