@@ -66,19 +66,21 @@ def test_other_dtypes(dtype, head_dim):
 # the fp32 sum's order leaves the scale an fp32 ulp off, an element crosses an
 # f16 rounding boundary (2^13 fp32 ulps apart) in 2^-13 of cases; an output takes
 # two elements and each a second rounding: at most 2^-11. (With a product's
-# rounding skipped, 0.12 of the elements differed.)
+# rounding skipped, 0.12 of the elements differed.) And every form gives the same
+# bits: the strided one's are those of the unit-stride one.
 @pytest.mark.parametrize("hq,hkv,head_dim", [(8, 2, 64), (8, 2, 128), (128, 8, 128), (4, 2, 256)])
-@pytest.mark.parametrize("strided", [False, True])
-def test_f16_rounding_points(hq, hkv, head_dim, strided):
-    w = W.make_prefill("f16", 13, 3, hq, hkv, 5, 40, dtype=torch.float16, head_dim=head_dim)
+def test_f16_rounding_points(hq, hkv, head_dim):
+    w = W.make_prefill("f16", 13, 3, hq, hkv, 60, 400, dtype=torch.float16, head_dim=head_dim)
     qr, kr = _oracle(w.q, w.k, w)
     q, k = w.q.to(DEV), w.k.to(DEV)
-    if strided:
-        q, k = (torch.stack([t, t], dim=-1)[..., 0] for t in (q, k))
-    qg, kg = qk_norm_rope(q, k, w.q_weight.to(DEV), w.k_weight.to(DEV), w.cos.to(DEV), w.sin.to(DEV), w.eps)
+    rest = [t.to(DEV) for t in (w.q_weight, w.k_weight, w.cos, w.sin)]
+    qg, kg = qk_norm_rope(q, k, *rest, w.eps)
+    qs, ks = qk_norm_rope(*(torch.stack([t, t], dim=-1)[..., 0] for t in (q, k)), *rest, w.eps)
     torch.cuda.synchronize()
     _check(qg, qr, "q", 2 ** -11)
     _check(kg, kr, "k", 2 ** -11)
+    assert_bitexact(qs, qg, "q, strided")
+    assert_bitexact(ks, kg, "k, strided")
 
 
 def test_strided_projection_views():

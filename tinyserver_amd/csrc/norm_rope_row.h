@@ -4,6 +4,8 @@
 // decode step, so both round identically.
 #pragma once
 
+#include <type_traits>
+
 #include "tsa_common.h"
 
 namespace tsa {
@@ -11,16 +13,16 @@ namespace tsa {
 template <typename T>
 __device__ __forceinline__ float round_t(float x) { return to_float(from_float<T>(x)); }
 
-// RoPE's product and sum, each with its own rounding for a 16-bit T. (__fmul_rn
-// and __fadd_rn are plain operators that may contract: in f16 the compiler
-// narrows a product that is rounded to f16 to the f16 multiply and fuses it
-// with the sum, in some kernels and not in others, so that one product is never
-// rounded: 12% of the outputs an ulp away from the model's. Uncontracted, the
-// fused step and the norm/RoPE kernels take the same time (f16, 8 sequences:
+// A product and a sum with a rounding of their own, for a 16-bit T. (__fmul_rn
+// and __fadd_rn are plain operators that may contract. In f16 the compiler then
+// narrows a product that is rounded to f16 to the f16 multiply and fuses it with
+// RoPE's sum, in some kernels and not in others, so that one product is never
+// rounded: 12% of the outputs were an ulp away from the model's. Uncontracted,
+// the fused step and the norm/RoPE kernels take the same time (f16, 8 sequences:
 // 21.8 us both ways; 16 packed prompts 71.3 and 71.5). bf16 has no such
 // multiply; in fp32 one rounding fewer is kept.)
 template <typename T>
-__device__ __forceinline__ float rope_mul(float x, float y) {
+__device__ __forceinline__ float mul_once(float x, float y) {
   if constexpr (sizeof(T) == 2) {
 #pragma clang fp contract(off)
     return x * y;
@@ -29,13 +31,23 @@ __device__ __forceinline__ float rope_mul(float x, float y) {
   }
 }
 template <typename T>
-__device__ __forceinline__ float rope_add(float x, float y) {
+__device__ __forceinline__ float add_once(float x, float y) {
   if constexpr (sizeof(T) == 2) {
 #pragma clang fp contract(off)
     return x + y;
   } else {
     return __fadd_rn(x, y);
   }
+}
+
+// x * rinv rounded to fp32, for a rounding to T that follows. (f16: behind an
+// opaque value, or the product and its rounding become one v_fma_mixlo_f16, which
+// rounds once, straight to f16: 6e-5 of the elements differed.)
+template <typename T>
+__device__ __forceinline__ float scaled(float x, float rinv) {
+  float y = mul_once<T>(x, rinv);
+  if constexpr (std::is_same<T, f16_t>::value) asm("" : "+v"(y));
+  return y;
 }
 
 // Cross-lane moves inside the 16-lane rows of a wave (DPP, no LDS traffic):
@@ -96,7 +108,7 @@ __device__ __forceinline__ void norm_rope_row(const float (&x)[8], const float (
 
   float z[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) z[i] = round_t<T>(__fmul_rn(wf[i], round_t<T>(__fmul_rn(x[i], rinv))));
+  for (int i = 0; i < 8; ++i) z[i] = round_t<T>(__fmul_rn(wf[i], round_t<T>(scaled<T>(x[i], rinv))));
 
   // Partner half: lane c holds dims 8c..8c+7, dims +- D/2 are in lane c ^ (LANES/2).
   float zp[8];
@@ -106,7 +118,7 @@ __device__ __forceinline__ void norm_rope_row(const float (&x)[8], const float (
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const float rot = first_half ? -zp[i] : zp[i];
-    o[i] = round_t<T>(rope_add<T>(round_t<T>(rope_mul<T>(z[i], cs[i])), round_t<T>(rope_mul<T>(rot, sn[i]))));
+    o[i] = round_t<T>(add_once<T>(round_t<T>(mul_once<T>(z[i], cs[i])), round_t<T>(mul_once<T>(rot, sn[i]))));
   }
 }
 
@@ -166,7 +178,7 @@ __device__ __forceinline__ void norm_rope_row_d128x8(const u32x4 (&xp)[2], const
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      float y0 = __fmul_rn(x[j][2 * i], rinv), y1 = __fmul_rn(x[j][2 * i + 1], rinv);
+      float y0 = scaled<T>(x[j][2 * i], rinv), y1 = scaled<T>(x[j][2 * i + 1], rinv);
       round2_t<T>(y0, y1);
       float z0 = __fmul_rn(lo_f<T>(wp[j][i]), y0), z1 = __fmul_rn(hi_f<T>(wp[j][i]), y1);
       round2_t<T>(z0, z1);
@@ -182,11 +194,11 @@ __device__ __forceinline__ void norm_rope_row_d128x8(const u32x4 (&xp)[2], const
       const float s0 = lo_f<T>(sp[j][i]), s1 = hi_f<T>(sp[j][i]);
       const float r0 = j == 0 ? -z[1][2 * i] : z[0][2 * i];
       const float r1 = j == 0 ? -z[1][2 * i + 1] : z[0][2 * i + 1];
-      float a0 = rope_mul<T>(z[j][2 * i], c0), a1 = rope_mul<T>(z[j][2 * i + 1], c1);
+      float a0 = mul_once<T>(z[j][2 * i], c0), a1 = mul_once<T>(z[j][2 * i + 1], c1);
       round2_t<T>(a0, a1);
-      float b0 = rope_mul<T>(r0, s0), b1 = rope_mul<T>(r1, s1);
+      float b0 = mul_once<T>(r0, s0), b1 = mul_once<T>(r1, s1);
       round2_t<T>(b0, b1);
-      op[j][i] = pack2<T>(rope_add<T>(a0, b0), rope_add<T>(a1, b1));
+      op[j][i] = pack2<T>(add_once<T>(a0, b0), add_once<T>(a1, b1));
     }
 }
 
