@@ -69,6 +69,11 @@ def test_page_ids_outside_the_pool_and_strided_rows(lens):
     (2, 2, 16, F16, [256, 257, 1, 512, 513, 700]),
     (8, 2, 256, BF, [1, 255, 257, 3000, 4096]),
     (8, 4, 16, BF, [8193, 64]),
+    # Past the unit form's limits (the stream), several tiles a wave: runs of
+    # one-tile units, more of them in flight than a wave has unit buffers.
+    (16, 8, 16, BF, [3000, 1, 17] * 7),
+    (8, 8, 32, F16, [3000] * 6 + [16] * 6 + [33, 1] * 6),
+    (2, 1, 16, BF, [33, 1, 17] * 501),             # the most sequences it takes
 ])
 def test_fused_step_is_the_two_launches(hq, hkv, page, dtype, lens):
     g = torch.Generator().manual_seed(hq + page)

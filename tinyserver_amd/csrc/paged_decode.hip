@@ -139,11 +139,14 @@ constexpr int kThreads = 64 * kWaves;
 #endif
 constexpr int RING = TSA_DECODE_RING;
 
-// Fused decode step: per wave, 1 KB of norm weights and RING unit buffers of
-// kUnitBytes in LDS after the tile prefixes. A unit buffer holds the raw q
+// Fused decode step: per wave, 1 KB of norm weights and kUnitBufs unit buffers
+// of kUnitBytes in LDS after the tile prefixes. A unit buffer holds the raw q
 // rows of its G <= 8 heads (2 KB), then the cos, sin, raw k and raw v rows of
-// the sequence's new token (256 B each at head_dim 128).
+// the sequence's new token (256 B each at head_dim 128). While a tile is
+// computed, the units of the RING tiles after it have been asked for, and each
+// may be a unit of its own: one buffer more than the ring has tiles.
 constexpr int kUnitBytes = 3072;
+constexpr int kUnitBufs = RING + 1;
 // The fused step's per-step values, kept in the wave's LDS area and read at
 // the unit events: held in scalar registers through the tile loop they
 // overflow them, and the spill reloads land in the loop.
@@ -153,7 +156,7 @@ struct FusedState {
   int64_t q_ss, q_sh, cs_ss, sn_ss, kn_ss, kn_sh, vn_ss, vn_sh;
   float eps;
 };
-constexpr int kStateOff = 1024 + RING * kUnitBytes;
+constexpr int kStateOff = 1024 + kUnitBufs * kUnitBytes;
 constexpr int kFusedWaveBytes = kStateOff + 128;
 static_assert(sizeof(FusedState) <= 128, "fused state exceeds its LDS slot");
 
@@ -578,7 +581,7 @@ __device__ __forceinline__ void decode_stream_body(DecodeArgs a, const int32_t* 
         ld.advance(pref, a.B, Hkv);
         --ld_left;
         if constexpr (FUSED) {
-          if (ld.t == 0) unit_dma(ld, ++ld_unit % RING);
+          if (ld.t == 0) unit_dma(ld, ++ld_unit % kUnitBufs);
         }
       }
     };
@@ -600,12 +603,12 @@ __device__ __forceinline__ void decode_stream_body(DecodeArgs a, const int32_t* 
             if (ustart || i + d == 0 || ulast) {
               // The tile's K/V have landed, so has this unit's LDS data.
               asm volatile("" ::"v"(kbuf[d][0]), "v"(vbuf[d][0]));
-              if (ustart || i + d == 0) make_q(cu_unit % RING);
+              if (ustart || i + d == 0) make_q(cu_unit % kUnitBufs);
             }
             if (ulast) {
               u32x4 kn[KJ], vnew;
               int cn;
-              new_token(cur, cu_unit % RING, kbuf[d], vbuf[d], kn, vnew, cn);
+              new_token(cur, cu_unit % kUnitBufs, kbuf[d], vbuf[d], kn, vnew, cn);
               compute_tile(cur, qn, kbuf[d], vbuf[d]);
               store_new_token(cur, kn, vnew, cn);
             } else {
@@ -937,6 +940,8 @@ static size_t fused_lds_bytes(int64_t B) {
   return ((static_cast<size_t>(kWaves) * (B + 1) * 4 + 15) & ~size_t(15)) +
          static_cast<size_t>(kWaves) * kFusedWaveBytes;
 }
+// Two such workgroups share a CU's 160 KB (1503 sequences).
+constexpr size_t kFusedMaxLds = 76 * 1024;
 
 template <typename T>
 static int launch_decode(DecodeArgs& a, bool mfma, hipStream_t stream, bool fused = false) {
@@ -1173,7 +1178,7 @@ static int prepare_decode_step(const tsa_view* out, const tsa_view* query, const
               "cos and sin must be (num_seqs, head_dim) of query's dtype");
   TSA_UNSUPPORTED(mfma && D == 128 && a.BS % 16 == 0 && a.kc_s == D && a.vc_s == D && a.G <= 8 &&
                       rows_vec16(k_new) && rows_vec16(v_new) && rows_vec16(q_weight) && rows_vec16(k_weight) &&
-                      rows_vec16(cos) && rows_vec16(sin) && fused_lds_bytes(B) <= 64 * 1024,
+                      rows_vec16(cos) && rows_vec16(sin) && fused_lds_bytes(B) <= kFusedMaxLds,
                   "the fused decode step needs a 16-bit dtype, head_dim 128, 16-token-multiple pages, contiguous "
                   "cache rows, at most 8 q-heads per kv head and unit-stride 16-byte-aligned rows");
   a.kn = k_new->data; a.vn = v_new->data; a.qw = q_weight->data; a.kw = k_weight->data;
