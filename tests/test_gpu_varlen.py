@@ -251,3 +251,21 @@ def test_groups_of_two_in_pairs(causal):
     assert torch.equal(torch.isnan(out), nan) and torch.equal(torch.isnan(one[:t]), nan)
     assert torch.equal(out[~nan], one[:t][~nan])
     assert_close(out[~nan], ref[~nan], what=f"pairs of 32-query blocks, causal={causal}")
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("lens", [[1000, 700, 65], [70, 100, 65]])
+def test_groups_of_two_bad_value_rows(lens, bad):
+    """Two q-heads per kv head, items of two 32-query blocks and of one (the
+    shorter sequences): a NaN or infinity in the V row of token t reaches
+    causal queries from t's own 32-token block on and none before it."""
+    q, k, v, cq, ck = _inputs(lens, lens, 16, 8, 128, torch.bfloat16, seed=53)
+    at = [cq[s] + t for s, t in enumerate((lens[0] // 64 * 64 - 10, lens[1] // 64 * 64 - 32, 33))]  # second blocks of a pair
+    args = [t.to(DEV) for t in (q, k)]
+    clean = flash_attn_varlen_func(*args, v.to(DEV), cq.to(DEV), ck.to(DEV), max(lens), max(lens), True).cpu()
+    v[torch.stack(at)] = bad
+    out = flash_attn_varlen_func(*args, v.to(DEV), cq.to(DEV), ck.to(DEV), max(lens), max(lens), True).cpu()
+    for s, n in enumerate(lens):
+        a, t = int(cq[s]), int(at[s] - cq[s])
+        assert torch.equal(out[a:a + t // 32 * 32], clean[a:a + t // 32 * 32]), (s, t)
+        assert not torch.isfinite(out[a + t:a + n]).any(), (s, t)

@@ -707,7 +707,10 @@ __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* _
     // X's last V block (whichever slot it is in) before they are issued.
     lds_barrier();
     if (nidx < n_items) load_head_v(Y);
-    if (X.nblk > 0) pv();
+    // (QS > 1: the item's last block can lie wholly after an earlier query block,
+    // whose wave leaves it out: its weights there are 0, but 0 times an infinity
+    // or NaN in V is NaN. So a bad V row reaches queries of its own 32 alone.)
+    if (X.nblk > 0 && !(QS > 1 && a.causal && 32 * j > X.q0 + 32 * my_blk)) pv();
     store_out(X);
     X = Y;
     idx = nidx;
