@@ -128,7 +128,8 @@ __device__ __forceinline__ void prefill_gqa_body(PrefillArgs a, const int32_t* _
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, c = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int HG = NW / QS, IQ = 32 * QS;  // q-heads of the group; queries of an item
-  const int my_head = wave % HG, my_blk = wave / HG;  // this wave's, within the item
+  // this wave's, within the item (QS = 1: the wave itself, which the compiler cannot tell from wave % NW)
+  const int my_head = QS == 1 ? wave : wave % HG, my_blk = QS == 1 ? 0 : wave / HG;
   const int nseq = a.nseq, Hkv = a.Hkv;
   const float cs = a.scale_log2;  // > 0 on this path
 
