@@ -69,3 +69,16 @@ def test_strided_rows_and_the_oracle(monkeypatch):
         for r in range(8):
             if got[r] != want[r]:  # only where the decision lies within 32-bit rounding of its target
                 assert os_.decision_margin(x[r], 0.9, 0, 0.8, float(un[r])) < 1e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_no_workspace_where_none_is_read(dtype):
+    """bf16 rows the key-count pass takes, and float32 rows, bring none (f16: 32 MB here)."""
+    x = torch.randn(64, 151936, device=DEV).to(dtype)
+    args = [torch.full((64,), val, dtype=dt, device=DEV) for val, dt in
+            ((1.0, torch.float32), (0, torch.int64), (0.95, torch.float32), (0.5, torch.float32))]
+    sample_tokens(x, *args)
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    sample_tokens(x, *args)
+    assert torch.cuda.max_memory_allocated() - before < 1 << 16

@@ -13,6 +13,8 @@ lies within fp32 rounding of a cumulative sum.
 
 from __future__ import annotations
 
+import os
+
 import torch
 
 from .. import _lib
@@ -53,7 +55,7 @@ def sample_tokens(
     if out is None:
         out = torch.empty(batch_size, dtype=torch.int64, device=dev)
     lib = _lib.load()
-    nbytes = _workspace_bytes(lib, *logits.shape)
+    nbytes = _workspace_bytes(lib, logits.dtype, *logits.shape)
     if nbytes:
         ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         rc = _lib.call("tsa_sample_tokens_ws", out, logits, temperature, top_k, top_p, uniforms, ws.data_ptr(), nbytes,
@@ -65,9 +67,16 @@ def sample_tokens(
 
 
 _WS_BYTES: dict = {}
+# Rows of up to this many bf16 logits are decided in one launch (sampling.hip:
+# kRegMaxV), unless the environment turns the passes that do so off.
+_ONE_LAUNCH_BF16 = 155648
 
 
-def _workspace_bytes(lib, batch: int, vocab: int) -> int:
+def _workspace_bytes(lib, dtype: torch.dtype, batch: int, vocab: int) -> int:
+    """The workspace worth bringing: 0 for rows that no split launch reads."""
+    if dtype == torch.float32 or (dtype == torch.bfloat16 and vocab <= _ONE_LAUNCH_BF16
+                                  and not os.environ.get("TSA_SAMPLE_CANDIDATES", "").startswith("0")):
+        return 0
     key = (batch, vocab)
     if key not in _WS_BYTES:
         _WS_BYTES[key] = int(lib.tsa_sample_tokens_workspace_bytes(batch, vocab))
