@@ -1,10 +1,11 @@
-"""The key-count pass of the sampler (bf16 rows of 16,384 to 155,648 logits)
-against the histogram paths (TSA_SAMPLE_CANDIDATES=0 in the environment): both
-add up the same integer masses and compare them with the same targets, so the
-tokens are equal, over the row's forms (vocabulary sizes at the ends of the
+"""The key-count pass of the sampler (bf16 rows of 16,384 to 155,648 logits; f16
+rows, which never take it, beside them) against the histogram paths
+(TSA_SAMPLE_CANDIDATES=0 in the environment): both add up the same integer masses
+and compare them with the same targets, so the tokens are equal, over the row's forms (vocabulary sizes at the ends of the
 range and beside a whole number of spans, heavy ties, both
 zeros, -inf and lowest-value masks, one value only, NaN, +inf), temperatures,
-top-k cuts above the candidate pass's and past the row's weight, top-p from 0
+top-k cuts of the candidate pass's (which sends rows of many ties on to the
+key-count pass), above them and past the row's weight, top-p from 0
 to past 1 and uniforms at both ends; and against the oracle in 64 bits."""
 
 import pytest
@@ -35,7 +36,7 @@ def _rows(v, dtype, seed):
 
 
 PARAMS = [(1.0, 0, 0.95), (1.0, 0, 1.0), (0.7, 600, 0.9), (1.3, 10 ** 6, 0.5), (0.05, 0, 0.999), (30.0, 5000, 1.5),
-          (1.0, 15000, 1.0), (1.0, 0, 0.0), (1e-5, 0, 0.9)]
+          (1.0, 15000, 1.0), (1.0, 0, 0.0), (1e-5, 0, 0.9), (0.8, 50, 0.9), (1.0, 512, 1.0), (1.0, 1, 1.0)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -82,3 +83,18 @@ def test_no_workspace_where_none_is_read(dtype):
     before = torch.cuda.memory_allocated()
     sample_tokens(x, *args)
     assert torch.cuda.max_memory_allocated() - before < 1 << 16
+
+
+@pytest.mark.parametrize("b", [3, 64, 86])
+def test_longer_rows_split(b):
+    """bf16 rows past the key-count pass's range: the split launches (with and
+    without bucket lists) against one workgroup a row (rows that start 2 bytes
+    off a 16-byte boundary)."""
+    g = torch.Generator().manual_seed(b)
+    v = 163840
+    x = (torch.randn(b, v, generator=g) * 2.5).to(torch.bfloat16).to(DEV)
+    odd = torch.empty(b, v + 8, dtype=torch.bfloat16, device=DEV)[:, 1:v + 1]
+    odd.copy_(x)
+    args = [torch.full((b,), val, dtype=dt, device=DEV) for val, dt in
+            ((1.0, torch.float32), (0, torch.int64), (0.95, torch.float32))] + [torch.rand(b, generator=g).to(DEV)]
+    assert sample_tokens(x, *args).tolist() == sample_tokens(odd, *args).tolist()
