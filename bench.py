@@ -257,16 +257,19 @@ def _decode_pools(w, copies):
 
 
 def _decode_kernels(w, page, num_workgroups):
-    """The launches of one decode call: a workspace of the tile prefix alone
-    (no partial slots) is the library's one-workgroup-per-unit form."""
-    from tinyserver_amd.kernels.paged_attention import decode_workspace_bytes
-
-    B = len(w.ctx_lens)
-    ws = decode_workspace_bytes(B, w.num_heads, w.num_kv_heads, w.q.shape[-1], w.block_tables.shape[1], page,
-                                num_workgroups)
-    if ws <= (4 * (B + 1) + 255) // 256 * 256:
+    """The launches of one decode call, by the limits of the library's plan
+    (paged_decode.hip, make_plan): the unit form for small block tables, one
+    workgroup a unit up to 32 tiles and one per 16 tiles above, else the stream."""
+    units = len(w.ctx_lens) * w.num_kv_heads
+    tiles = -(-w.block_tables.shape[1] * page // 16)
+    splits = 1 if tiles <= 32 else -(-tiles // 16)
+    limit = 768 if splits == 1 else 1024 if splits < 32 else 2048
+    part_bytes = units * splits * (w.num_heads // w.num_kv_heads) * (w.q.shape[-1] + 2) * 4
+    if num_workgroups or units * splits > limit or (splits > 1 and part_bytes > 15 << 20):
+        return "paged_decode_stream + paged_decode_stream_merge"
+    if splits == 1:
         return "paged_decode_unit (one workgroup per unit, no merge launch)"
-    return "paged_decode_stream + paged_decode_stream_merge"
+    return "paged_decode_unit (split units) + decode_split_merge"
 
 
 def bench_decode(name, steps, warmup, num_workgroups=0, copies=3, with_block=False, **make_kw):

@@ -186,7 +186,7 @@ int tsa_paged_decode_noalloc(const tsa_view* out, const tsa_view* query, const t
                              void* stream);
 /* The decode step of the Qwen3 call site, fused (qwen3.py:268-287 norm and
  * RoPE of q and of the new k, :335-357 the store of the new token's k and v,
- * :359-409 paged_attention_forward), in the two launches of tsa_paged_decode:
+ * :359-409 paged_attention_forward), in the launches of tsa_paged_decode:
  * query (B, Hq, D) and k / v (B, Hkv, D) are the raw projections of each
  * sequence's new token, at position seq_lens[s] - 1; q_weight, k_weight (D);
  * cos / sin (B, D) for those positions. The rotated k and the raw v are

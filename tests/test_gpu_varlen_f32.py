@@ -1,6 +1,6 @@
 """The float32 varlen prefill kernel (f32 matrix instructions) against 64-bit
 softmax attention: tile and key-block edges (a tile is 32 (query, head) rows,
-a key block 32 keys, dealt to four waves), GQA groups that do and do not
+a key block 16 keys, dealt to four waves), GQA groups that do and do not
 divide 32, q_len != k_len, more than 64 sequences (the other item order), a
 sequence without keys, and non-finite V rows that no query may see through
 the causal mask. Tolerance: an output is a mean of the V rows, whose 32-bit

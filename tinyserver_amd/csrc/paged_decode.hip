@@ -48,8 +48,9 @@
 //   runs cover it with a log-sum-exp reduce. The kernel boundary orders the
 //   two, so no cache flushes or atomics are needed; no host sync, no memset.
 // * Batches of small block tables take the unit form instead
-//   (paged_decode_unit.h): one workgroup per 512 tokens of a unit, with no
-//   prefix, and no merge launch where a unit has one workgroup.
+//   (paged_decode_unit.h), with no prefix: one workgroup a unit and no merge
+//   launch for tables of up to 512 tokens, above that one per 256 tokens and a
+//   merge.
 //
 // Tokens past seq_len are scored -inf and their V rows zeroed (the
 // reference's masked loads, :88-105). seq_len is clamped to the block table's
@@ -1087,9 +1088,10 @@ static int check_decode(const tsa_view* out, const tsa_view* query, const tsa_vi
     a.NW = kWaves * plan.W;
     a.S = plan.S;
   } else if (dt == TSA_F32 && rows_vec16(query) && rows_vec16(k_cache) && rows_vec16(v_cache) && decode_f32_takes(a)) {
-    // The partials of its splits fit the plan's slots, so the workspace the
-    // caller was told to bring serves (the one-workgroup-per-unit form has no
-    // slots: one split).
+    // The partials of its splits fit the slots of the 16-bit plan for these
+    // sizes, so the workspace the caller was told to bring serves. Where that
+    // plan has no slots (at most kUnitNoSlots units, tables of up to 512 tokens)
+    // a unit is one split.
     plan = make_plan(B, Hq, Hkv, D, block_tables->size[1], BS, num_workgroups);
     const int64_t units = B * Hkv;
     a.S = units == 0 ? 1 : decode_f32_splits(units, (block_tables->size[1] * BS + 15) / 16,
@@ -1232,13 +1234,16 @@ constexpr int kMixedLds = gqa_smem_bytes<128, 4>();
 // Sharing a CU, the two roles slow each other down -- the LDS-staged
 // prefill's loads wait behind the decode's HBM stream -- so one launch pays
 // only when both halves are small. Measured on Qwen3-4B heads, one kernel vs
-// the two launches, both replayed from a captured graph:
-//   4 decode (ctx 128-512) + 322 prefill tokens        23.1 vs 26.7 us
-//   16 decode (ctx 256-2048) + 365 prefill tokens      30.3 vs 35.4 us
-//   32 decode (ctx 256-4096) + 402 prefill tokens      67.5 vs 70.7 us
-//   64 decode (ctx 256-4096) + 402 prefill tokens     118.9 vs 117.9 us
-//   120 decode (ctx 256-8192) + 402 prefill tokens    350.3 vs 339.6 us
-//   120 decode (ctx 256-8192) + 5760 prefill tokens   436.1 vs 402.0 us
+// the two launches, both replayed from a captured graph (span: the block tables'
+// tokens; the first three decode halves take the unit form):
+//   4 decode (ctx 128-512, span 1,728) + 322 prefill tokens       10.4 vs 20.2 us
+//   8 decode (ctx 128-512, span 3,584) + 400                      11.3 vs 22.3
+//   16 decode (ctx 256-2048, span 32,512) + 365                   28.5 vs 34.2
+//   32 decode (ctx 256-2048, span 64,512) + 400                   42.8 vs 50.0
+//   32 decode (ctx 256-4096, span 130,048) + 402                  68.7 vs 73.0
+//   64 decode (ctx 256-4096, span 262,144) + 402                 109.6 vs 109.4
+//   120 decode (ctx 256-8192, span 979,200) + 402                345.2 vs 332.0
+//   120 decode (ctx 256-8192, span 979,200) + 5760               436.4 vs 399.8
 constexpr int64_t kMixedAutoMaxTokens = 512;
 constexpr int64_t kMixedAutoMaxDecodeTokens = 131072;
 static_assert(kMixedLds >= 64 * 1024, "the mixed kernel's LDS also holds the decode tile prefixes (at most 64 KB)");

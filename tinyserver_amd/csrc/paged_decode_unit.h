@@ -11,8 +11,8 @@
 // exponential pass, no rescaling, and pairs of tiles share the 32-token form of
 // the P V product. Wave w takes tiles w, w + 8, w + 16 and w + 24 of the 32.
 // The waves' partials meet in LDS. A unit of more than 32 tiles is split over
-// S workgroups, which leave one partial each for a merge launch
-// (decode_split_merge).
+// S workgroups of four waves and 16 tiles (256 tokens), which leave one partial
+// each for a merge launch (decode_split_merge).
 //
 // Measured against the form before it (four waves a unit, one tile at a time
 // through a register ring, three tiles ahead; the fused step staged its rows
@@ -21,8 +21,9 @@
 // x 256-512 12.1 -> 8.5. Against the stream and its merge: 32 x 64-512, 32/8
 // heads, 18.8 -> 12.6; fused step of 8 x 128-4096, 16/8 heads, 26.8 -> 22.5
 // (70 MB of K/V, 14 us at a large copy's rate). Splits of eight waves took
-// 24.9 there: at 153 registers one such workgroup fills a CU, where three of
-// four waves overlap.
+// 24.9 there: at the fused step's 173 registers (two waves a SIMD) one such
+// workgroup fills a CU, where two of four waves overlap. (The plain form has 153:
+// three waves a SIMD.)
 //
 // The fused step adds the norm and RoPE of the unit's q rows and of the new
 // token's k row: 16 lanes a row, four rows a wave, in the first waves, while

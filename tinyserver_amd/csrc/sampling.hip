@@ -45,7 +45,11 @@
 // it replaces for these rows (151,936 logits): 64 rows at the server's default
 // request 47 -> 28 us, 8 mixed rows 36 -> 26, 256 rows 103 -> 38, rows of one
 // value 995 -> 147; top-k and greedy rows, which needed neither launch, 17 ->
-// 13 (eager).
+// 13 (eager). A launch that takes it splits no row, so a row it refuses is left
+// to one workgroup: NaN and +inf rows lose nothing by that (8 rows, one of them
+// such, 39 -> 27), finite rows spanning over 36,864 values (logits past 2^17 on
+// both sides of 0 at a temperature past 9,000) do (8 rows 36 -> 76, 64 rows 46 ->
+// 83).
 #include <cmath>
 #include <cstdlib>
 #include <type_traits>
@@ -2211,9 +2215,9 @@ __global__ __launch_bounds__(kSampThreads) void sample_tokens_kernel(SampleArgs 
   // while the row arrives. (top_k as its low and high words, with no branch
   // on its type between the loads.) An f16 row may be one that the split
   // launches have read, whose merge would wait behind a load that nothing uses
-  // (64 rows, server default: 48.6 us with it, 46.6 without; 8 mixed rows 36.7
-  // and 34.7), so f16 rows are loaded once that is known. A bf16 row that fits
-  // the registers is never one.
+  // (64 rows, server default: 48.2 us with it, 45.6 without; 8 mixed rows 36.4
+  // and 34.3), or one for the histogram path (300 rows 155 and 146), so f16 rows
+  // are loaded once that is known. A bf16 row that fits the registers is neither.
   const float temp = a.temp[r * a.temp_s], pf = a.topp[r * a.topp_s], uf = a.unif[r * a.unif_s];
   const int wide_k = a.topk_dt == TSA_I64 ? 1 : 0;
   const int32_t* const k32 = static_cast<const int32_t*>(a.topk) + ((r * a.topk_s) << wide_k);

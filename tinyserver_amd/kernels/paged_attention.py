@@ -125,7 +125,8 @@ def paged_decode_step(
     out: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """One decode step of the Qwen3 attention layer: QK RMSNorm + RoPE of the
-    new token, its paged K/V store, and paged attention, in two launches.
+    new token, its paged K/V store, and paged attention, in one launch or, where
+    units are split (tables above 512 tokens, large batches), with a merge launch.
 
     q (B, Hq, D), k and v (B, Hkv, D) are the raw projections of each
     sequence's new token, at position ``seq_lens[s] - 1``; cos/sin (B, D) are

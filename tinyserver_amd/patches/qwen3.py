@@ -167,12 +167,15 @@ def device_metadata(ctx: Any, position_ids: torch.Tensor | None, num_tokens: int
 # A decode step whose KV spans at most this many 16-token tiles (per kv head
 # summed over the heads) takes the single-launch fused step; larger ones take
 # the norm/store launch followed by paged attention. The fused kernel saves a
-# launch (a few microseconds) but pays at every (sequence, kv head) unit it
-# enters (the unit's loads into LDS, its norm, a wait for them), which
-# outweighs the saved launch on large steps. Measured at head_dim 128 on 256
-# CUs: Qwen3-0.6B batch 4 (550 tiles) 29 us fused vs 50 us; Qwen3-8B batch 64
-# (74k tiles) 131 us vs 132 us; a 120-sequence batch (257k tiles) 394 us vs
-# 357 us.
+# launch (a few microseconds); past the unit form's limits it pays at every
+# (sequence, kv head) unit it enters (the unit's loads into LDS, its norm, a
+# wait for them), which outweighs the saved launch. Measured at head_dim 128 on
+# 256 CUs, replayed, fused vs two launches: 4 x 16-512 tokens, 16/8 heads (432
+# tiles) 7.7 vs 10.7 us; 64 x 16-512 (9,504) 20.1 vs 22.6; 8 x 128-4096 (9,856)
+# 22.8 vs 24.9; 16 x 256-2048, 32/8 heads (10,344) 24.7 vs 25.9 -- all the unit
+# form; beyond it 48 x 200-700 (11,008) 31.8 vs 31.6, 32 x 256-2048 (16,280) 40.8
+# vs 37.4, 64 x 512-4096 (67,592) 115.7 vs 100.6, 120 x 256-8192 (256,632) 396 vs
+# 336, and many short units the most: 100 x 16-300 (8,408) 35.3 vs 26.5.
 FUSED_DECODE_MAX_TILES = 16384
 
 
