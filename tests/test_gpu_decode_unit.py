@@ -3,8 +3,9 @@ a unit up to 512 tokens, splits of 256 tokens above) against 64-bit softmax
 attention: tile, wave and split edges, GQA groups of 1 to 16, head_dim 64 and
 128, pages of 4 to 256 tokens, strided cache rows, an empty sequence, page ids
 outside the pool, non-finite slots past a sequence's end, tables on both sides
-of the plan's limits; the fused step with its new token at those edges and the
-one-launch prefill + decode, both bit-identical to the calls they stand for.
+of the plan's limits; the fused step with its new token at those edges (and past
+them, in the stream) and the one-launch prefill + decode, both bit-identical to
+the calls they stand for.
 Tolerance: the output is rounded to its type (bf16: 2^-9 of the value, f16:
 2^-12), P keeps 16 (22) bits, so 2^-8 (2^-11) of values of order 1."""
 
